@@ -122,6 +122,9 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream);
 // row offset of the pool fits in 32 bits).
 bool decode_ws_takes(const DecodeParams& p);
 hipError_t launch_decode_ws(const DecodeParams& p, hipStream_t stream);
+// The few-heads kernel: up to 32 heads, any power-of-two page size (with the same bound on the pool).
+bool decode_fh_takes(const DecodeParams& p);
+hipError_t launch_decode_fh(const DecodeParams& p, hipStream_t stream);
 hipError_t launch_merge(const MergeParams& p, hipStream_t stream);
 hipError_t launch_store_rows(void* cache, int64_t cache_rows, int64_t cache_stride, const void* x, int64_t x_stride,
                              const void* indices, int index_bits, int64_t rows, int64_t row_bytes,

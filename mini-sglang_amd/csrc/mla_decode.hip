@@ -429,6 +429,7 @@ hipError_t launch_decode_nw(const DecodeParams& p, hipStream_t stream) {
 
 hipError_t launch_decode(const DecodeParams& p, hipStream_t stream) {
   if (decode_ws_takes(p)) return launch_decode_ws(p, stream);
+  if (decode_fh_takes(p)) return launch_decode_fh(p, stream);
   if (p.heads < 1 || p.heads > 64) return hipErrorInvalidValue;  // the entry points split larger counts
   switch ((p.heads + 15) / 16) {
     case 1: return launch_decode_nw<1>(p, stream);

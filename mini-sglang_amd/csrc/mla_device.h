@@ -1,6 +1,8 @@
 // Device helpers shared by the gfx950 MLA decode kernels.
 #pragma once
 
+#include <type_traits>
+
 #include "mla_common.h"
 
 namespace mla {
@@ -9,16 +11,41 @@ namespace mla {
 // position c ^ swz(t & 7).
 __device__ __forceinline__ int swz(int t7) { return ((t7 & 3) << 1) | ((t7 >> 2) & 1); }
 
+// Combines a lane's value with lanes l ^ 16, l ^ 32 and l ^ 48 (the four lane groups; every lane gets the
+// result) by v_permlane16_swap / v_permlane32_swap: no LDS traffic and no LDS latency.
+template <typename F>
+__device__ __forceinline__ float group_reduce(float v, F&& f) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = f(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return f(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
 __device__ __forceinline__ float wave_max_g(float v) {
-  // reduce over the 4 lane groups (lanes l, l^16, l^32, l^48)
-  v = fmaxf(v, __shfl_xor(v, 16));
-  v = fmaxf(v, __shfl_xor(v, 32));
-  return v;
+  return group_reduce(v, [](float a, float b) { return fmaxf(a, b); });
 }
 __device__ __forceinline__ float wave_sum_g(float v) {
-  v += __shfl_xor(v, 16);
-  v += __shfl_xor(v, 32);
-  return v;
+  return group_reduce(v, [](float a, float b) { return a + b; });
+}
+
+// A lane's value combined over the whole wave (every lane gets the result): four row rotations by DPP, then
+// the group swaps: a dozen vector instructions, where six ds_bpermute steps wait out the LDS latency each.
+template <typename F>
+__device__ __forceinline__ float wave_reduce(float v, F&& f) {
+  auto ror = [&](auto ctrl) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), decltype(ctrl)::value,
+                                                                  0xf, 0xf, false));
+  };
+  v = f(v, ror(std::integral_constant<int, 0x128>{}));  // row_ror:8
+  v = f(v, ror(std::integral_constant<int, 0x124>{}));
+  v = f(v, ror(std::integral_constant<int, 0x122>{}));
+  v = f(v, ror(std::integral_constant<int, 0x121>{}));
+  return group_reduce(v, f);
+}
+__device__ __forceinline__ float wave_max64(float v) {
+  return wave_reduce(v, [](float a, float b) { return fmaxf(a, b); });
+}
+__device__ __forceinline__ float wave_sum64(float v) {
+  return wave_reduce(v, [](float a, float b) { return a + b; });
 }
 
 // Wait until at most N vector-memory operations of this wave are outstanding.

@@ -12,12 +12,6 @@ namespace {
 constexpr int kRopeDim = 64;
 constexpr int kNopeDim = 128;
 
-__device__ __forceinline__ float wave_sum64(float v) {
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o);
-  return v;
-}
-
 __device__ __forceinline__ void unpack8(const u32x4 w, float (&f)[8]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) {

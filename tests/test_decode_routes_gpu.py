@@ -1,0 +1,89 @@
+"""Head counts and page sizes at the edges of the decode dispatch, against the CPU oracle.
+
+Up to 16 heads run the few-heads kernel unless pages are under 32 tokens and the pool's row offsets do not
+fit in 32 bits (then the general kernel). Tolerances: bf16 output atol = rtol = 2e-2, fp32
+LSE atol 1e-3 (as everywhere in the decode tests).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from minisgl_amd.benchmark.inputs import make_decode_case
+from minisgl_amd.kernel import lib
+from oracle import ref_mla as R
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+O_TOL = dict(atol=2e-2, rtol=2e-2)
+LSE_TOL = dict(atol=1e-3, rtol=0.0)
+
+
+def _decode(q, kv, pt, lens, ps, num_ctas, spare_slots=0):
+    B, H, _ = q.shape
+    plan_np, slots = lib.decode_plan(lens, ps, num_ctas)
+    ws_o, ws_lse = lib.decode_workspace(slots + spare_slots, H, DEV)
+    # one more head than the call's: its rows must stay untouched
+    out = torch.full((B, H + 1, 512), 7.0, dtype=torch.bfloat16, device=DEV)
+    lse = torch.full((B, H + 1), 7.0, dtype=torch.float32, device=DEV)
+    lib.mla_decode(q.to(DEV), kv.to(DEV), pt.to(DEV), torch.tensor(lens, dtype=torch.int32, device=DEV),
+                   torch.from_numpy(plan_np).to(DEV), num_ctas, ws_o, ws_lse, R.DEFAULT_SCALE, out[:, :H], lse[:, :H])
+    torch.cuda.synchronize()
+    assert torch.all(out[:, H] == 7.0) and torch.all(lse[:, H] == 7.0)
+    return out[:, :H].cpu(), lse[:, :H].cpu()
+
+
+@pytest.mark.parametrize("heads,ps,num_ctas", [
+    (1, 64, 300), (16, 1, 7), (16, 128, 400), (5, 8, 2), (17, 64, 64), (80, 1, 16),
+])
+def test_decode_dispatch_edges(heads, ps, num_ctas):
+    """Empty requests first, last and in between; pieces shorter than a tile; more ranges than compute units."""
+    print(f"[decode edges] heads={heads} ps={ps} ctas={num_ctas}", flush=True)
+    lens = [0, 1, 31, 0, 33, 700, 2049, 64, 0]
+    case = make_decode_case(len(lens), heads, ps, lens=lens, seed=heads + ps)
+    out, lse = _decode(case.q, case.kv_pool, case.page_table, lens, ps, num_ctas)
+    o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, lens)
+    full = torch.tensor([L > 0 for L in lens])
+    torch.testing.assert_close(out[full].float(), o_ref[full], **O_TOL)
+    torch.testing.assert_close(lse[full], lse_ref[full], **LSE_TOL)
+    assert torch.all(out[~full] == 0) and torch.all(torch.isneginf(lse[~full]))
+
+
+@pytest.mark.parametrize("heads,ps", [(8, 64), (8, 1)])
+def test_decode_growing_logits(heads, ps):
+    """Scores that pass the piece's exponent reference by more than 2^64, several times over."""
+    case = make_decode_case(2, heads, ps, lens=[900, 2000], seed=29)
+    kv = case.kv_pool.float()
+    for b, L in enumerate(case.lens):  # grows along each request
+        rows = R.token_rows(case.page_table[b], L, ps)
+        kv.view(-1, 576)[rows, 512] = torch.linspace(0, 160.0, L)
+    case.kv_pool = kv.to(torch.bfloat16)
+    case.q[..., 512] = 20.0
+    out, lse = _decode(case.q, case.kv_pool, case.page_table, case.lens, ps, 8)
+    o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, case.lens)
+    torch.testing.assert_close(out.float(), o_ref, **O_TOL)
+    torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
+
+
+def test_decode_head_counts_beyond_32_bit_offsets():
+    """A page-size-1 pool of more than 4 GiB: every head count takes the general kernel."""
+    pages = (1 << 32) // 1152 + 4096
+    lens = [300, 77]
+    g = torch.Generator().manual_seed(41)
+    pool = torch.empty((pages, 1, 576), dtype=torch.bfloat16, device=DEV)
+    rows = torch.randn((1000, 1, 576), generator=g).to(torch.bfloat16)
+    pool[:500] = rows[:500].to(DEV)
+    pool[pages - 500 :] = rows[500:].to(DEV)
+    perm = torch.randperm(1000, generator=g)
+    small_pt = torch.zeros((2, 300), dtype=torch.int32)
+    small_pt[0] = perm[:300].to(torch.int32)
+    small_pt[1, :77] = perm[300:377].to(torch.int32)
+    pt = torch.where(small_pt < 500, small_pt, small_pt - 1000 + pages)
+    for heads in (5, 20, 40, 70):
+        q = torch.randn((2, heads, 576), generator=g).to(torch.bfloat16)
+        o_ref, lse_ref = R.mla_decode(q, rows, small_pt, lens)
+        out, lse = _decode(q, pool, pt, lens, 1, 12)
+        torch.testing.assert_close(out.float(), o_ref, **O_TOL)
+        torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
