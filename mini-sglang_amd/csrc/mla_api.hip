@@ -280,7 +280,6 @@ static int decode_params(const char* who, const void* q, int64_t q_stride_b, int
                          int32_t heads, float scale, const int32_t* plan, int32_t num_ctas, __bf16* ws_o,
                          float* ws_lse, int32_t ws_slots, void* out, int64_t out_stride_b, int64_t out_stride_h,
                          float* lse, int64_t lse_stride_b, mla::DecodeParams* p) {
-  if (heads < 1 || heads > 64) return fail(MLA_ERR_UNSUPPORTED, "%s: heads must be in [1, 64], got %d", who, heads);
   if (q == nullptr || kv_pool == nullptr || page_table == nullptr || seq_lens == nullptr || plan == nullptr)
     return fail(MLA_ERR_INVALID_ARG, "%s: null pointer", who);
   if (!aligned(q, 16) || q_stride_h % 8 != 0 || q_stride_b % 8 != 0 || q_stride_h < MLA_KV_DIM ||
@@ -371,6 +370,31 @@ static HeadGroup head_group(int32_t h0, int32_t heads, int32_t ws_slots, const v
   return g;
 }
 
+// One launch of all heads where the kernel takes them (it runs the groups itself), else one per group.
+static int decode_launches(const char* who, const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* kv_pool,
+                           int64_t kv_row_stride, int32_t num_pages, int32_t page_size, const int32_t* page_table,
+                           int64_t pt_stride, const int32_t* seq_lens, int32_t batch, int32_t heads, float scale,
+                           const int32_t* plan, int32_t num_ctas, __bf16* ws_o, float* ws_lse, int32_t ws_slots, void* out,
+                           int64_t out_stride_b, int64_t out_stride_h, float* lse, int64_t lse_stride_b, void* stream) {
+  mla::DecodeParams p;
+  if (int rc = decode_params(who, q, q_stride_b, q_stride_h, kv_pool, kv_row_stride, num_pages, page_size, page_table,
+                             pt_stride, seq_lens, batch, heads, scale, plan, num_ctas, ws_o, ws_lse, ws_slots, out,
+                             out_stride_b, out_stride_h, lse, lse_stride_b, &p))
+    return rc;
+  if (heads <= kHeadGroup || mla::decode_ws_takes(p)) return hip_status(mla::launch_decode(p, (hipStream_t)stream), who);
+  for (int32_t h0 = 0; h0 < heads; h0 += kHeadGroup) {
+    const HeadGroup g = head_group(h0, heads, ws_slots, q, q_stride_h, ws_o, ws_lse, out, out_stride_h, lse);
+    p.q = static_cast<const __bf16*>(g.q);
+    p.ws_o = g.ws_o;
+    p.ws_lse = g.ws_lse;
+    p.out = static_cast<__bf16*>(g.out);
+    p.lse = g.lse;
+    p.heads = g.heads;
+    if (int rc = hip_status(mla::launch_decode(p, (hipStream_t)stream), who)) return rc;
+  }
+  return ok();
+}
+
 static int check_head_groups(const char* who, int32_t heads, int64_t q_stride_b, int64_t q_stride_h,
                              int64_t out_stride_b, int64_t out_stride_h, const float* lse, int64_t lse_stride_b) {
   if (heads < 1 || heads > kMaxHeads) return fail(MLA_ERR_UNSUPPORTED, "%s: heads must be in [1, %d], got %d", who, kMaxHeads, heads);
@@ -391,16 +415,9 @@ int mla_decode_split_bf16(const void* q, int64_t q_stride_b, int64_t q_stride_h,
   if (batch == 0) return ok();
   if (int rc = check_head_groups(who, heads, q_stride_b, q_stride_h, out_stride_b, out_stride_h, lse, lse_stride_b))
     return rc;
-  for (int32_t h0 = 0; h0 < heads; h0 += kHeadGroup) {
-    const HeadGroup g = head_group(h0, heads, ws_slots, q, q_stride_h, static_cast<__bf16*>(ws_o), ws_lse, out, out_stride_h, lse);
-    mla::DecodeParams p;
-    if (int rc = decode_params(who, g.q, q_stride_b, q_stride_h, kv_pool, kv_row_stride, num_pages, page_size,
-                               page_table, pt_stride, seq_lens, batch, g.heads, scale, plan, num_ctas, g.ws_o,
-                               g.ws_lse, ws_slots, g.out, out_stride_b, out_stride_h, g.lse, lse_stride_b, &p))
-      return rc;
-    if (int rc = hip_status(mla::launch_decode(p, (hipStream_t)stream), "mla_decode_split_bf16 launch")) return rc;
-  }
-  return ok();
+  return decode_launches(who, q, q_stride_b, q_stride_h, kv_pool, kv_row_stride, num_pages, page_size, page_table,
+                         pt_stride, seq_lens, batch, heads, scale, plan, num_ctas, static_cast<__bf16*>(ws_o), ws_lse,
+                         ws_slots, out, out_stride_b, out_stride_h, lse, lse_stride_b, stream);
 }
 
 int mla_decode_bf16(const void* q, int64_t q_stride_b, int64_t q_stride_h, const void* kv_pool,
@@ -449,20 +466,13 @@ int decode_split_merge(const char* who, const void* q, int64_t q_stride_b, int64
   if (batch == 0) return ok();
   if (int rc = check_head_groups(who, heads, q_stride_b, q_stride_h, out_stride_b, out_stride_h, lse, lse_stride_b))
     return rc;
-  for (int32_t h0 = 0; h0 < heads; h0 += kHeadGroup) {
-    const HeadGroup g = head_group(h0, heads, ws_slots, q, q_stride_h, ws_o, ws_lse, out, out_stride_h, lse);
-    mla::DecodeParams p;
-    if (int rc = decode_params(who, g.q, q_stride_b, q_stride_h, kv_pool, kv_row_stride, num_pages, page_size,
-                               page_table, pt_stride, seq_lens, batch, g.heads, scale, plan, num_ctas, g.ws_o,
-                               g.ws_lse, ws_slots, g.out, out_stride_b, out_stride_h, g.lse, lse_stride_b, &p))
-      return rc;
-    hipError_t e = mla::launch_decode(p, (hipStream_t)stream);
-    if (e != hipSuccess) return hip_status(e, "decode split launch");
-    const mla::MergeParams m = merge_params(g.ws_o, g.ws_lse, ws_slots, plan + 4 * (int64_t)num_ctas, batch, g.heads,
-                                            1, g.out, out_stride_b, out_stride_h, g.lse, lse_stride_b);
-    if (int rc = hip_status(mla::launch_merge(m, (hipStream_t)stream), "decode merge launch")) return rc;
-  }
-  return ok();
+  if (int rc = decode_launches(who, q, q_stride_b, q_stride_h, kv_pool, kv_row_stride, num_pages, page_size, page_table,
+                               pt_stride, seq_lens, batch, heads, scale, plan, num_ctas, ws_o, ws_lse, ws_slots, out,
+                               out_stride_b, out_stride_h, lse, lse_stride_b, stream))
+    return rc;
+  const MergeParams m = merge_params(ws_o, ws_lse, ws_slots, plan + 4 * (int64_t)num_ctas, batch, heads, 1, out,
+                                     out_stride_b, out_stride_h, lse, lse_stride_b);
+  return hip_status(mla::launch_merge(m, (hipStream_t)stream), "decode merge launch");
 }
 
 }  // namespace mla
@@ -479,15 +489,10 @@ int mla_decode_merge_f32(const void* ws_o, const float* ws_lse, int32_t ws_slots
     return fail(MLA_ERR_INVALID_ARG, "%s: null pointer", who);
   if (ws_o != nullptr && !aligned(ws_o, 16)) return fail(MLA_ERR_INVALID_ARG, "%s: ws_o must be 16-byte aligned", who);
   if (int rc = check_out(out, out_stride_b, out_stride_h, lse, lse_stride_b, heads, who)) return rc;
-  for (int32_t h0 = 0; h0 < heads; h0 += kHeadGroup) {  // the workspace holds one [slots, group, 512] block per group
-    const HeadGroup g = head_group(h0, heads, ws_slots, nullptr, 0, static_cast<__bf16*>(const_cast<void*>(ws_o)),
-                                   const_cast<float*>(ws_lse), out, out_stride_h, lse);
-    const mla::MergeParams m = merge_params(g.ws_o, g.ws_lse, ws_slots, req_info, batch, g.heads,
-                                            single_piece_final ? 1 : 0, g.out, out_stride_b, out_stride_h, g.lse,
-                                            lse_stride_b);
-    if (int rc = hip_status(mla::launch_merge(m, (hipStream_t)stream), "mla_decode_merge_f32 launch")) return rc;
-  }
-  return ok();
+  const mla::MergeParams m =
+      merge_params(static_cast<const __bf16*>(ws_o), ws_lse, ws_slots, req_info, batch, heads, single_piece_final ? 1 : 0,
+                   out, out_stride_b, out_stride_h, lse, lse_stride_b);
+  return hip_status(mla::launch_merge(m, (hipStream_t)stream), "mla_decode_merge_f32 launch");
 }
 
 // Shared checks and launch of the prefill entry points; K/V rows as in mla::PrefillParams.

@@ -1,5 +1,9 @@
-// Absorbed-MLA paged decode for gfx950 (MI355X), split-KV, plus the fp32
-// log-sum-exp merge of the split partials (bf16 partial outputs, fp32 LSEs).
+// Absorbed-MLA paged decode for gfx950 (MI355X), split-KV: the general kernel, plus the fp32 log-sum-exp
+// merge of the split partials (bf16 partial outputs, fp32 LSEs).
+//
+// The general kernel runs what neither the few-heads kernel (up to 16 heads) nor the warp-specialized one
+// (17 heads and more) takes: pages of fewer than 32 tokens in a pool past 4 GiB, whose row offsets need 64
+// bits.
 //
 // Work decomposition: a CTA (one wave per 16 query heads) owns one contiguous
 // range of (request, 64-token block) space from the host plan. For each piece
@@ -41,7 +45,7 @@ constexpr int kKPrefetch = 8;  // K operands (16-byte LDS reads) in flight
 constexpr int kVPrefetch = 4;  // V operand pairs (transposing LDS reads) in flight
 constexpr int kQkChains = 3;   // independent QK accumulators per 16-token block
 
-template <int NW, bool kPageCoversTile>
+template <int NW>
 __global__ __launch_bounds__(NW * 64, 1) void mla_decode_kernel(const DecodeParams p) {
   constexpr int kDmaPerWave = kTileDma / NW;
   static_assert(kTileDma % NW == 0, "tile DMA split");
@@ -81,12 +85,6 @@ __global__ __launch_bounds__(NW * 64, 1) void mla_decode_kernel(const DecodePara
     auto slot_chunk16 = [&](int k, int t) {
       return (((wave + k * NW) * 64 + lane - t * kRowChunks) ^ swz(t & 7)) << 4;
     };
-    uint32_t dma_voff[kDmaPerWave];  // byte offset of this lane's chunk from the tile's first row
-#pragma unroll
-    for (int k = 0; k < kDmaPerWave; ++k) {
-      const int t = slot_token(k);
-      dma_voff[k] = t * row_bytes + slot_chunk16(k, t);
-    }
 
     for (int b = rb; b <= re && b < p.batch; ++b) {
       const int L = p.seq_lens[b];
@@ -145,28 +143,13 @@ __global__ __launch_bounds__(NW * 64, 1) void mla_decode_kernel(const DecodePara
         const int tlim = t1 - 1 - tstart;  // last valid token of the tile (loads clamp to it)
         const uint32_t lds_stage = lds_ring + stage * kTileBytes;
         const int id0 = pg0 + win * kMaxPieceIds;  // page of s_ids[0]
-        if constexpr (kPageCoversTile) {
-          const int pid = __builtin_amdgcn_readfirstlane(s_ids[(tstart >> p.log2_ps) - id0]);
-          const char* tsrc = kv + ((int64_t)pid * (ps_mask + 1) + (tstart & ps_mask)) * row_bytes;
-          if (tlim >= kTile - 1) {
 #pragma unroll
-            for (int k = 0; k < kDmaPerWave; ++k) dma16_saddr(tsrc, dma_voff[k], lds_stage + (wave + k * NW) * 1024);
-          } else {
-#pragma unroll
-            for (int k = 0; k < kDmaPerWave; ++k) {
-              const int t = slot_token(k);
-              dma16_saddr(tsrc, min(t, tlim) * row_bytes + slot_chunk16(k, t), lds_stage + (wave + k * NW) * 1024);
-            }
-          }
-        } else {
-#pragma unroll
-          for (int k = 0; k < kDmaPerWave; ++k) {
-            const int t = slot_token(k);
-            const int tok = tstart + min(t, tlim);
-            const int pid = s_ids[(tok >> p.log2_ps) - id0];
-            const char* src = kv + ((int64_t)pid * (ps_mask + 1) + (tok & ps_mask)) * row_bytes + slot_chunk16(k, t);
-            dma16_vaddr(src, lds_stage + (wave + k * NW) * 1024);
-          }
+        for (int k = 0; k < kDmaPerWave; ++k) {
+          const int t = slot_token(k);
+          const int tok = tstart + min(t, tlim);
+          const int pid = s_ids[(tok >> p.log2_ps) - id0];
+          const char* src = kv + ((int64_t)pid * (ps_mask + 1) + (tok & ps_mask)) * row_bytes + slot_chunk16(k, t);
+          dma16_vaddr(src, lds_stage + (wave + k * NW) * 1024);
         }
       };
 
@@ -329,13 +312,20 @@ __global__ __launch_bounds__(NW * 64, 1) void mla_decode_kernel(const DecodePara
   }
 }
 
-// One wave per (request, head). Lane l reads 16-byte chunk l of every piece's bf16 partial row
-// (value dims 32 (l / 4) + 4 (l % 4) + {0..3, 16..19}, the chunk order of mla_amd.h) and the LSE of
-// piece l (of each group of 64 pieces). The first kMergeBatch pieces are requested together with the
-// LSEs, so a request of up to 8 pieces costs one memory round trip; later pieces are read 8 at a
-// time. Each piece's weight exp(lse_i - lse) is computed once, by lane i, and read by the wave
-// with v_readlane. fp32 arithmetic, one rounding to bf16.
+// Merge of one (request, head): kWaves waves (1: four heads per CTA; 4: one head per CTA), wave v of them
+// takes pieces v, v + kWaves, ... Lane l reads 16-byte chunk l of a piece's bf16 partial row (value dims
+// 32 (l / 4) + 4 (l % 4) + {0..3, 16..19}, the chunk order of mla_amd.h) and the LSE of piece l (of each
+// group of 64 pieces). A wave's first kMergeBatch pieces are requested together with the LSEs, so a request of
+// up to 8 kWaves pieces costs one memory round trip after its plan entry's; later pieces are read 8 at a time.
+// Each piece's weight exp(lse_i - lse) is computed once, by lane i, and read by the wave with v_readlane. fp32
+// arithmetic, one rounding to bf16; piece i is added to partial sum i % 4 for either kWaves, so both give the
+// same bits.
+// Bound: latency (launch, plan entry, partials, output), so four waves pay where a request has more pieces
+// than one wave reads in a round trip. Step time less the split step's, 64 heads: one request in 23 pieces
+// 8.3 -> 3.8 us, 8 of 1k to 8k tokens 11.3 -> 5.4 us, 8 of 32k to 128k tokens 9.9 -> 3.9 us; at 8 slots per
+// request (32 requests, 128 heads) one wave is the faster by 1.4 us, at 10.7 (24 requests) four by 1.3 us.
 constexpr int kMergeBatch = 8;
+constexpr int kMergeWideSlots = 10;  // workspace slots per request from which four waves merge a head
 
 __device__ __forceinline__ void unpack_bf16x8(const u32x4 raw, float* f) {
 #pragma unroll
@@ -345,9 +335,13 @@ __device__ __forceinline__ void unpack_bf16x8(const u32x4 raw, float* f) {
   }
 }
 
+template <int kWaves>
 __global__ __launch_bounds__(256) void mla_merge_kernel(const MergeParams p) {
+  __shared__ __attribute__((aligned(16))) f32x4 s_acc[kWaves > 1 ? kWaves - 1 : 1][2][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int b = blockIdx.x;
-  const int h = blockIdx.y * 4 + (threadIdx.x >> 6);
+  const int h = kWaves == 1 ? blockIdx.y * 4 + wave : blockIdx.y;
+  const int v = kWaves == 1 ? 0 : wave;
   const int lane = threadIdx.x & 63;
   if (h >= p.heads) return;
   const int n = p.req_info[3 * b + 1];
@@ -356,72 +350,94 @@ __global__ __launch_bounds__(256) void mla_merge_kernel(const MergeParams p) {
   // slots outside the workspace (a caller's plan that does not match it) give NaN, never a silent result
   const bool in_ws = n <= 0 || (base >= 0 && (int64_t)base + n <= p.ws_slots);
   const int nv = in_ws && n > 0 ? n : 0;
-  const __bf16* src = p.ws_o + ((int64_t)(nv > 0 ? base : 0) * p.heads + h) * kVDim + 8 * lane;
-  const int64_t pstride = (int64_t)p.heads * kVDim;
-  auto piece_lse = [&](int i) { return p.ws_lse[(int64_t)(base + i) * p.heads + h]; };
+  // the head's 64-head group: its partials are a [ws_slots, group heads, 512] block of the workspace
+  const int h0 = h & ~63, gh = min(64, p.heads - h0);
+  const int64_t slot0 = nv > 0 ? base : 0;
+  const __bf16* src = p.ws_o + ((int64_t)p.ws_slots * h0 + slot0 * gh + (h - h0)) * kVDim + 8 * lane;
+  const float* src_lse = p.ws_lse + (int64_t)p.ws_slots * h0 + slot0 * gh + (h - h0);
+  const int64_t pstride = (int64_t)gh * kVDim;
+  auto piece_lse = [&](int i) { return src_lse[(int64_t)i * gh]; };
   u32x4 raw[kMergeBatch];
 #pragma unroll
   for (int u = 0; u < kMergeBatch; ++u)
-    if (u < nv) raw[u] = *reinterpret_cast<const u32x4*>(src + u * pstride);
+    if (v + kWaves * u < nv) raw[u] = *reinterpret_cast<const u32x4*>(src + (v + kWaves * u) * pstride);
   const float lse0 = lane < nv ? piece_lse(lane) : -INFINITY;
 
   constexpr float kLog2e = 1.4426950408889634f;
   float mx = lse0;
   for (int i = lane + 64; i < nv; i += 64) mx = fmaxf(mx, piece_lse(i));
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+  mx = wave_max64(mx);
   float sum = 0.f;
   if (mx > -INFINITY) {
     sum = lse0 > -INFINITY ? __builtin_amdgcn_exp2f((lse0 - mx) * kLog2e) : 0.f;
     for (int i = lane + 64; i < nv; i += 64) sum += __builtin_amdgcn_exp2f((piece_lse(i) - mx) * kLog2e);
   }
-#pragma unroll
-  for (int o = 32; o >= 1; o >>= 1) sum += __shfl_xor(sum, o);
+  sum = wave_sum64(sum);
   const bool any = mx > -INFINITY && sum > 0.f;
   const float lse = any ? mx + logf(sum) : -INFINITY;
 
-  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  constexpr int kAcc = 4 / kWaves;  // partial sums of this wave: pieces i with i % 4 == v + a (kWaves 1: v = 0)
+  float acc[kAcc][8];
+#pragma unroll
+  for (int a = 0; a < kAcc; ++a)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[a][j] = 0.f;
   if (any) {
+    // rounds of kMergeBatch pieces of this wave; 64 pieces' weights at a time
 #pragma unroll 1
     for (int i0 = 0; i0 < nv; i0 += 64) {
       const float l_i = i0 == 0 ? lse0 : (i0 + lane < nv ? piece_lse(i0 + lane) : -INFINITY);
       const float w_i = l_i > -INFINITY ? __builtin_amdgcn_exp2f((l_i - lse) * kLog2e) : 0.f;  // lane u: piece i0 + u
       const int cnt = min(64, nv - i0);
 #pragma unroll 1
-      for (int u0 = 0; u0 < cnt; u0 += kMergeBatch) {
+      for (int u0 = 0; u0 < cnt; u0 += kMergeBatch * kWaves) {
         if (i0 + u0 > 0) {
 #pragma unroll
           for (int u = 0; u < kMergeBatch; ++u)
-            if (u0 + u < cnt) raw[u] = *reinterpret_cast<const u32x4*>(src + (i0 + u0 + u) * pstride);
+            if (u0 + v + kWaves * u < cnt)
+              raw[u] = *reinterpret_cast<const u32x4*>(src + (i0 + u0 + v + kWaves * u) * pstride);
         }
 #pragma unroll
         for (int u = 0; u < kMergeBatch; ++u) {
-          if (u0 + u < cnt) {
-            const float wgt = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w_i), u0 + u));
+          const int i = u0 + v + kWaves * u;
+          if (i < cnt) {
+            const float wgt = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w_i), i));
             float f[8];
             unpack_bf16x8(raw[u], f);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] = fmaf(wgt, f[j], acc[j]);
+            for (int j = 0; j < 8; ++j) acc[u % kAcc][j] = fmaf(wgt, f[j], acc[u % kAcc][j]);
           }
         }
       }
     }
   }
+  float o[8];
+  if constexpr (kWaves == 1) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = (acc[0][j] + acc[1][j]) + (acc[2][j] + acc[3][j]);
+  } else {
+    if (v > 0) {
+      s_acc[v - 1][0][lane] = f32x4{acc[0][0], acc[0][1], acc[0][2], acc[0][3]};
+      s_acc[v - 1][1][lane] = f32x4{acc[0][4], acc[0][5], acc[0][6], acc[0][7]};
+    }
+    __syncthreads();
+    if (v > 0) return;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      o[j] = (acc[0][j] + s_acc[0][j >> 2][lane][j & 3]) +
+             (s_acc[kWaves > 2 ? 1 : 0][j >> 2][lane][j & 3] + s_acc[kWaves > 2 ? 2 : 0][j >> 2][lane][j & 3]);
+  }
   const float bad = in_ws ? 0.f : __builtin_nanf("");
   __bf16* orow = p.out + (int64_t)b * p.out_stride_b + (int64_t)h * p.out_stride_h + 32 * (lane >> 2) + 4 * (lane & 3);
-  *reinterpret_cast<u32x2*>(orow) = u32x2{pack_bf16x2(acc[0] + bad, acc[1] + bad), pack_bf16x2(acc[2] + bad, acc[3] + bad)};
-  *reinterpret_cast<u32x2*>(orow + 16) =
-      u32x2{pack_bf16x2(acc[4] + bad, acc[5] + bad), pack_bf16x2(acc[6] + bad, acc[7] + bad)};
+  *reinterpret_cast<u32x2*>(orow) = u32x2{pack_bf16x2(o[0] + bad, o[1] + bad), pack_bf16x2(o[2] + bad, o[3] + bad)};
+  *reinterpret_cast<u32x2*>(orow + 16) = u32x2{pack_bf16x2(o[4] + bad, o[5] + bad), pack_bf16x2(o[6] + bad, o[7] + bad)};
   if (p.lse != nullptr && lane == 0) p.lse[(int64_t)b * p.lse_stride_b + h] = lse + bad;
 }
 
 template <int NW>
 hipError_t launch_decode_nw(const DecodeParams& p, hipStream_t stream) {
   const int grid = p.num_ctas < current_device_cus() ? p.num_ctas : current_device_cus();
-  if (p.log2_ps >= 5)
-    hipLaunchKernelGGL((mla_decode_kernel<NW, true>), dim3(grid), dim3(NW * 64), 0, stream, p);
-  else
-    hipLaunchKernelGGL((mla_decode_kernel<NW, false>), dim3(grid), dim3(NW * 64), 0, stream, p);
+  hipLaunchKernelGGL(mla_decode_kernel<NW>, dim3(grid), dim3(NW * 64), 0, stream, p);
   return hipGetLastError();
 }
 
@@ -441,8 +457,11 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream) {
 }
 
 hipError_t launch_merge(const MergeParams& p, hipStream_t stream) {
-  dim3 grid(p.batch, (p.heads + 3) / 4);
-  hipLaunchKernelGGL(mla_merge_kernel, grid, dim3(256), 0, stream, p);
+  // The plan is on the device; the workspace's slots bound the pieces of an average request.
+  if ((int64_t)p.ws_slots >= (int64_t)kMergeWideSlots * p.batch && p.heads <= 65535)
+    hipLaunchKernelGGL(mla_merge_kernel<4>, dim3(p.batch, p.heads), dim3(256), 0, stream, p);
+  else
+    hipLaunchKernelGGL(mla_merge_kernel<1>, dim3(p.batch, (p.heads + 3) / 4), dim3(256), 0, stream, p);
   return hipGetLastError();
 }
 

@@ -1,5 +1,5 @@
-// Warp-specialized absorbed-MLA decode for 64 query heads and pages of >= 32 tokens (the Kimi-K2 /
-// DeepSeek-V3 decode shape on one GPU). Same plan, workspace and outputs as mla_decode_kernel.
+// Warp-specialized absorbed-MLA decode for 17 heads and more (the Kimi-K2 / DeepSeek-V3 decode shapes), in
+// groups of 64, any page size. Same plan, workspace and outputs as mla_decode_kernel.
 //
 //  * The CTA's whole (request, token) range is one stream of 32-row tiles: per piece, two tiles of
 //    queries (heads 0..31, 32..63; a query row has the latent row's 576 dims, so it is staged like
@@ -65,8 +65,47 @@ struct WCursor {
 // first padding range. Without it (at most one range per compute unit) each CTA runs range blockIdx.x
 // and the body has no loop around it: the loop makes the compiler keep values across both roles'
 // step loops and spill.
-template <bool kSmall, bool kLoop>
-__global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const DecodeParams p) {
+// kMode kPadded: 17 to 63 heads; query rows past the last head load the last head again and their outputs are
+// not written (the padding costs MFMAs, which the KV stream hides: 32 heads, 64 requests of 1k to 8k tokens,
+// 67.9 us against 78.1 us on the general kernel; 48 heads 70.7 against 82.5 us). kMode kGroups: more than 64 heads, in groups of 64 (the last one padded): CTA
+// blockIdx.x runs one group of one range, and the groups of a range are CTAs 8 apart, which the dispatcher
+// puts on the same XCD at about the same time: the range's KV tiles come from HBM once and from that XCD's
+// L2 for the other groups (so they are loaded without the non-temporal hint). One launch per group, each
+// streaming the KV from HBM, took 80.8 us for 128 heads, 32 requests of 1k to 8k tokens; this takes 77.2 us
+// (the step is then bound by the waves' own chain of loads, MFMAs and barriers, no longer by HBM).
+enum WMode { kExact, kPadded, kGroups };
+
+template <bool kSmall, bool kLoop, WMode kMode>
+__global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const DecodeParams p0) {
+  DecodeParams p = p0;
+  int w_first = blockIdx.x;
+  if constexpr (kMode == kGroups) {
+    const int groups = (p0.heads + 63) >> 6;
+    const int i = (int)blockIdx.x >> 3, grp = i % groups;
+    w_first = (i / groups) * 8 + ((int)blockIdx.x & 7);
+    if (w_first >= p0.num_ctas) return;
+    const int h0 = 64 * grp;
+    p.heads = min(64, p0.heads - h0);
+    p.q = p0.q + (int64_t)h0 * p0.q_stride_h;
+    p.ws_o = p0.ws_o + (int64_t)p0.ws_slots * h0 * kVDim;  // the group's own [ws_slots, group heads] block
+    p.ws_lse = p0.ws_lse + (int64_t)p0.ws_slots * h0;
+    p.out = p0.out + (int64_t)h0 * p0.out_stride_h;
+    if (p0.lse != nullptr) p.lse = p0.lse + h0;
+  }
+  // a DMA load of KV rows: non-temporal where they are read once
+  auto dma_kv = [&](const char* base, uint32_t voff, uint32_t lds) __attribute__((always_inline)) {
+    if constexpr (kMode == kGroups) dma16_saddr(base, voff, lds);
+    else dma16_saddr_nt(base, voff, lds);
+  };
+  // first query row of query tile qt, and row t of it from there (rows past the last head: the last head)
+  auto q_tile_row = [&](int qt) __attribute__((always_inline)) {
+    return kMode == kExact ? 32 * qt : min(32 * qt, p.heads - 1);
+  };
+  auto q_row = [&](int t, int qt) __attribute__((always_inline)) {
+    return kMode == kExact ? t : min(t, p.heads - 1 - q_tile_row(qt));
+  };
+  // head blocks of 16 with a head in them: the stores of an output wave are counted for these
+  const int hblocks = kMode == kExact ? 4 : (p.heads + 15) >> 4;
   __shared__ __attribute__((aligned(1024))) char smem[kStages * kTileBytes];
   // softmax numerators of the last two scored tiles: [tile parity][head block][lane], 16 B per lane
   __shared__ __attribute__((aligned(16))) u32x4 s_p[2][4][64];
@@ -126,13 +165,13 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) {
         const char* qsrc = reinterpret_cast<const char*>(p.q) +
-                           ((int64_t)rb * p.q_stride_b + (int64_t)(32 * qt) * p.q_stride_h) * 2;
+                           ((int64_t)rb * p.q_stride_b + (int64_t)q_tile_row(qt) * p.q_stride_h) * 2;
 #pragma unroll
         for (int k = 0; k < kWOutParts; ++k) {
           const int part = 4 * kWScoreParts + role + 4 * k;
           const int s = part * 64 + lane;
           const int t = (s * 7282) >> 19;  // s / 72
-          dma16_saddr(qsrc, t * qrow_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
+          dma16_saddr(qsrc, q_row(t, qt) * qrow_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
                       lds_ring + qt * kTileBytes + part * 1024);
         }
       }
@@ -236,21 +275,21 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
       if (cur.q < 2) {  // query rows 32q .. +32 of request rb + r
         const int qrow_bytes = (int)(p.q_stride_h * 2);
         const char* qsrc = reinterpret_cast<const char*>(p.q) +
-                           ((int64_t)(rb + cur.r) * p.q_stride_b + (int64_t)(32 * cur.q) * p.q_stride_h) * 2;
+                           ((int64_t)(rb + cur.r) * p.q_stride_b + (int64_t)q_tile_row(cur.q) * p.q_stride_h) * 2;
         int ln;  // lane index from a volatile asm, so these offsets are computed here
         asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
 #pragma unroll
         for (int k = 0; k < nparts; ++k) {
           const int s = (part0 + 4 * k) * 64 + ln;
           const int t = (s * 7282) >> 19;
-          dma16_saddr(qsrc, t * qrow_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
+          dma16_saddr(qsrc, q_row(t, cur.q) * qrow_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
                       stage + (part0 + 4 * k) * 1024);
         }
       } else if constexpr (kSmall) {  // each lane's token row from the offset ring (clamped rows included)
         const int ring = (n & 3) * 32;
 #pragma unroll
         for (int k = 0; k < nparts; ++k)
-          dma16_saddr_nt(kv, (uint32_t)s_pid[ring + (dma_voff[k] >> 16)] + (dma_voff[k] & 0xffff),
+          dma_kv(kv, (uint32_t)s_pid[ring + (dma_voff[k] >> 16)] + (dma_voff[k] & 0xffff),
                          stage + (part0 + 4 * k) * 1024);
       } else {
         const int pid = __builtin_amdgcn_readfirstlane(s_pid[min(iss_kv++, kWMaxTiles - 1)]);
@@ -258,7 +297,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
         const int tlim = cur.t1 - 1 - cur.t;  // loads clamp to the piece's last token
         if (tlim >= kTile - 1) {
 #pragma unroll
-          for (int k = 0; k < nparts; ++k) dma16_saddr_nt(tsrc, dma_voff[k], stage + (part0 + 4 * k) * 1024);
+          for (int k = 0; k < nparts; ++k) dma_kv(tsrc, dma_voff[k], stage + (part0 + 4 * k) * 1024);
         } else {
           int ln;
           asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
@@ -266,7 +305,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
           for (int k = 0; k < nparts; ++k) {
             const int s = (part0 + 4 * k) * 64 + ln;
             const int t = (s * 7282) >> 19;
-            dma16_saddr_nt(tsrc, min(t, tlim) * row_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
+            dma_kv(tsrc, min(t, tlim) * row_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
                            stage + (part0 + 4 * k) * 1024);
           }
         }
@@ -487,9 +526,10 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
               if (valid < kTile && 16 * th + 4 * g + i >= valid) x[hb][i] = -INFINITY;
               mt[hb] = fmaxf(mt[hb], x[hb][i]);
             }
-            mt[hb] = wave_max_g(mt[hb]);  // this head's max over this half of the tile
           }
           if (first_kv && attempt == 0) {
+            mt[0] = wave_max_g(mt[0]);  // each head's max over this half of the tile
+            mt[1] = wave_max_g(mt[1]);
             // the piece's reference: the first tile's max over both halves, agreed with the wave that
             // holds the other half (an extra barrier, which every wave takes at this step; the output
             // waves are idle here, the previous tile being a query tile)
@@ -507,7 +547,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
           u32x2 pown[2];
 #pragma unroll
           for (int hb = 0; hb < 2; ++hb) {
-            m_max[hb] = fmaxf(m_max[hb], mt[hb]);
+            m_max[hb] = fmaxf(m_max[hb], mt[hb]);  // (over this lane's tokens; reduced when the piece ends)
             overflow |= mt[hb] > m_ref[hb] + kWOverflowLog2;
             float pr[4];
 #pragma unroll
@@ -529,10 +569,11 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
 #pragma unroll
             for (int hb = 0; hb < 2; ++hb) {
               const float l_half = wave_sum_g(l_run[hb]);
+              const float m_half = wave_max_g(m_max[hb]);
               const int h = 32 * hg + 16 * hb + c;
               if (g == 0) {
                 s_l[th][h] = l_half;
-                s_mx[th][h] = m_max[hb];
+                s_mx[th][h] = m_half;
                 if (th == 0) s_mref[h] = m_ref[hb];
               }
               m_max[hb] = -INFINITY;
@@ -587,6 +628,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
 #pragma unroll
             for (int hq = 0; hq < 4; ++hq) {
               const int h = 16 * hq + c;
+              if (kMode != kExact && h >= p.heads) continue;
               const float l = s_l[0][h] + s_l[1][h];
               const float inv = l > 0.f ? 1.f / l : 0.f;
               if (to_ws) {
@@ -613,19 +655,22 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
                 }
               }
             }
-            ops += to_ws ? 16 : 32;
+            ops += (to_ws ? 4 : 8) * hblocks;
             // the LSE of head block `role`
             const int h = 16 * role + c;
             const float l = s_l[0][h] + s_l[1][h];
             const float lse_nat = l > 0.f ? (s_mref[h] + log2f(l)) * 0.69314718055994531f : -INFINITY;
-            if (!to_ws) {
-              if (p.lse != nullptr) {
-                if (g == 0) p.lse[(int64_t)b * p.lse_stride_b + h] = lse_nat;
+            if (role < hblocks) {
+              const bool h_ok = kMode == kExact || h < p.heads;
+              if (!to_ws) {
+                if (p.lse != nullptr) {
+                  if (g == 0 && h_ok) p.lse[(int64_t)b * p.lse_stride_b + h] = lse_nat;
+                  ops += 1;
+                }
+              } else {
+                if (g == 0 && h_ok) p.ws_lse[(int64_t)slot * p.heads + h] = lse_nat;
                 ops += 1;
               }
-            } else {
-              if (g == 0) p.ws_lse[(int64_t)slot * p.heads + h] = lse_nat;
-              ops += 1;
             }
           }
 #pragma unroll
@@ -667,14 +712,14 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
       if (!range(w)) break;
     }
   } else {
-    range(blockIdx.x);
+    range(w_first);
   }
 }
 
 }  // namespace
 
 bool decode_ws_takes(const DecodeParams& p) {
-  if (p.heads != 64) return false;
+  if (p.heads <= 16) return false;
   if (p.log2_ps >= 5) return true;
   // pages under 32 tokens: every row offset from the pool base must fit in 32 bits
   return ((int64_t)p.num_pages << p.log2_ps) * p.kv_row_stride * 2 <= (int64_t)UINT32_MAX;
@@ -683,10 +728,17 @@ bool decode_ws_takes(const DecodeParams& p) {
 template <bool kSmall>
 static void launch_ws(const DecodeParams& p, hipStream_t stream) {
   const int cus = current_device_cus();
-  if (p.num_ctas <= cus)
-    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, false>), dim3(p.num_ctas), dim3(kWWaves * 64), 0, stream, p);
-  else
-    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, true>), dim3(cus), dim3(kWWaves * 64), 0, stream, p);
+  const dim3 threads(kWWaves * 64);
+  if (p.heads > 64) {  // one CTA per (range, 64-head group); ranges in eights (one per XCD)
+    const int grid = (p.num_ctas + 7) / 8 * 8 * ((p.heads + 63) / 64);
+    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, false, kGroups>), dim3(grid), threads, 0, stream, p);
+  } else if (p.heads < 64) {
+    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, false, kPadded>), dim3(p.num_ctas), threads, 0, stream, p);
+  } else if (p.num_ctas <= cus) {
+    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, false, kExact>), dim3(p.num_ctas), threads, 0, stream, p);
+  } else {
+    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, true, kExact>), dim3(cus), threads, 0, stream, p);
+  }
 }
 
 hipError_t launch_decode_ws(const DecodeParams& p, hipStream_t stream) {

@@ -1,7 +1,8 @@
 """Head counts and page sizes at the edges of the decode dispatch, against the CPU oracle.
 
-Up to 16 heads run the few-heads kernel unless pages are under 32 tokens and the pool's row offsets do not
-fit in 32 bits (then the general kernel). Tolerances: bf16 output atol = rtol = 2e-2, fp32
+Up to 16 heads run the few-heads kernel, 17..63 the warp-specialized kernel padded to 64, more than 64 its
+groups of 64 in one launch (the last group padded), and any count the general kernel when pages are under
+32 tokens and the pool's row offsets do not fit in 32 bits. Tolerances: bf16 output atol = rtol = 2e-2, fp32
 LSE atol 1e-3 (as everywhere in the decode tests).
 """
 
@@ -36,7 +37,8 @@ def _decode(q, kv, pt, lens, ps, num_ctas, spare_slots=0):
 
 
 @pytest.mark.parametrize("heads,ps,num_ctas", [
-    (1, 64, 300), (16, 1, 7), (16, 128, 400), (5, 8, 2), (17, 64, 64), (80, 1, 16),
+    (1, 64, 300), (16, 1, 7), (16, 128, 400), (5, 8, 2), (17, 64, 64), (33, 1, 64), (47, 32, 300), (63, 4, 5),
+    (65, 64, 64), (80, 1, 16), (127, 64, 300), (130, 16, 9),
 ])
 def test_decode_dispatch_edges(heads, ps, num_ctas):
     """Empty requests first, last and in between; pieces shorter than a tile; more ranges than compute units."""
@@ -51,7 +53,7 @@ def test_decode_dispatch_edges(heads, ps, num_ctas):
     assert torch.all(out[~full] == 0) and torch.all(torch.isneginf(lse[~full]))
 
 
-@pytest.mark.parametrize("heads,ps", [(8, 64), (8, 1)])
+@pytest.mark.parametrize("heads,ps", [(8, 64), (8, 1), (24, 64), (70, 8)])
 def test_decode_growing_logits(heads, ps):
     """Scores that pass the piece's exponent reference by more than 2^64, several times over."""
     case = make_decode_case(2, heads, ps, lens=[900, 2000], seed=29)
@@ -67,8 +69,36 @@ def test_decode_growing_logits(heads, ps):
     torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
 
 
+@pytest.mark.parametrize("heads,L,num_ctas", [(3, 64 * 9, 9), (8, 64 * 33 + 5, 40), (66, 64 * 70, 70), (64, 64 * 200, 200)])
+def test_decode_merge_widths_give_the_same_bits(heads, L, num_ctas):
+    """One request in many pieces, merged by four waves per head and, with a second request's slots spread
+    over a batch of short ones, by one wave: the same partials give the same bits either way."""
+    case = make_decode_case(1, heads, 64, lens=[L], seed=heads)
+    plan, slots = lib.decode_plan([L], 64, num_ctas)
+    assert slots >= num_ctas // 2
+    wide = _decode(case.q, case.kv_pool, case.page_table, [L], 64, num_ctas)
+    o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, [L])
+    torch.testing.assert_close(wide[0].float(), o_ref, **O_TOL)
+    torch.testing.assert_close(wide[1], lse_ref, **LSE_TOL)
+    # the same partials merged in a batch of `slots` requests (one slot per request on average: one wave)
+    ws_o, ws_lse = lib.decode_workspace(slots, heads, DEV)
+    out = torch.empty((slots, heads, 512), dtype=torch.bfloat16, device=DEV)
+    lse = torch.empty((slots, heads), dtype=torch.float32, device=DEV)
+    plan_dev = torch.from_numpy(plan).to(DEV)
+    lib.mla_decode(case.q.to(DEV), case.kv_pool.to(DEV), case.page_table.to(DEV),
+                   torch.tensor([L], dtype=torch.int32, device=DEV), plan_dev, num_ctas, ws_o, ws_lse, R.DEFAULT_SCALE,
+                   out[:1], lse[:1], split_only=True)
+    info = plan_dev[num_ctas * 4 :].view(1, 3).expand(slots, 3).contiguous()
+    lib.mla_decode_merge(ws_o, ws_lse, info, out, lse)
+    torch.cuda.synchronize()
+    for b in (0, slots - 1):
+        assert torch.equal(out[b].cpu().view(torch.int16), wide[0][0].view(torch.int16))
+        assert torch.equal(lse[b].cpu(), wide[1][0])
+
+
 def test_decode_head_counts_beyond_32_bit_offsets():
-    """A page-size-1 pool of more than 4 GiB: every head count takes the general kernel."""
+    """A page-size-1 pool of more than 4 GiB: every head count takes the general kernel, above 64 heads in
+    one launch per group."""
     pages = (1 << 32) // 1152 + 4096
     lens = [300, 77]
     g = torch.Generator().manual_seed(41)
