@@ -45,9 +45,15 @@ __global__ __launch_bounds__(256) void page_table_kernel(const int32_t* __restri
 // Latent rows of every key of a prefill batch into 64-row scratch pages, the input of the per-head
 // decompression: key j of request b (pool row pt[b, j >> log2_ps] * ps + (j & (ps - 1)), page ids
 // clamped into the pool) goes to scratch row 64 seg_first[b] + j, its 512 latent dims to c_out and
-// its 64 rope dims to rope_out; the scratch page table gets seg_pt[b, i] = seg_first[b] + i. CTA
-// (i, b) copies scratch page i of request b: 64 rows x 72 16-byte chunks, consecutive threads on
-// consecutive chunks of a row. Rows at or past out_rows are not written.
+// its 64 rope dims to rope_out; the scratch page table gets seg_pt[b, i] = seg_first[b] + i. Rows at or
+// past out_rows are not written.
+// Bound: latency (a few MB). CTA (i, b) copies kGatherRows rows, 72 16-byte chunks each, consecutive threads
+// on consecutive chunks: the rows' page ids go to LDS in one round trip, then every thread has all its
+// chunks in flight at once. (A 64-row CTA whose threads looked a page id up for each of their 18 chunks,
+// one after the other, took 22.4 us for 4.7k keys at page size 1.)
+constexpr int kGatherRows = 16;
+constexpr int kGatherChunks = (kGatherRows * kRowChunks + 255) / 256;  // per thread
+
 __global__ __launch_bounds__(256) void prefill_gather_kernel(const char* __restrict__ kv, int64_t kv_row_bytes,
                                                              int32_t num_pages, int32_t log2_ps,
                                                              const int32_t* __restrict__ page_table, int64_t pt_stride,
@@ -57,27 +63,35 @@ __global__ __launch_bounds__(256) void prefill_gather_kernel(const char* __restr
                                                              char* __restrict__ rope_out, int64_t rope_row_bytes,
                                                              int64_t out_rows, int32_t* __restrict__ seg_pt,
                                                              int64_t seg_pt_stride) {
+  __shared__ int64_t s_src[kGatherRows];
   const int b = blockIdx.y;
-  const int pg = blockIdx.x;
   const int L = seq_lens_k[b];
-  const int j0 = pg * 64;
+  const int j0 = blockIdx.x * kGatherRows;
   if (j0 >= L) return;
   const int first = seg_first[b];
-  if (threadIdx.x == 0) seg_pt[(int64_t)b * seg_pt_stride + pg] = first + pg;
-  const int rows = min(64, L - j0);
-  const int ps_mask = (1 << log2_ps) - 1;
-  for (int i = threadIdx.x; i < rows * 72; i += 256) {
-    const int r = i / 72, ch = i - 72 * r;
-    const int j = j0 + r;
-    const int64_t dst = (int64_t)first * 64 + j;
-    if (dst < 0 || dst >= out_rows) continue;
+  const int rows = min(kGatherRows, L - j0);
+  if ((int)threadIdx.x < rows) {
+    const int j = j0 + threadIdx.x;
     const int pid = min(max(page_table[(int64_t)b * pt_stride + (j >> log2_ps)], 0), num_pages - 1);
-    const int64_t src = ((int64_t)pid << log2_ps) + (j & ps_mask);
-    const u32x4 v = *reinterpret_cast<const u32x4*>(kv + src * kv_row_bytes + ch * 16);
+    s_src[threadIdx.x] = (((int64_t)pid << log2_ps) + (j & ((1 << log2_ps) - 1))) * kv_row_bytes;
+  }
+  if (threadIdx.x == 0 && j0 % 64 == 0) seg_pt[(int64_t)b * seg_pt_stride + j0 / 64] = first + j0 / 64;
+  __syncthreads();
+  u32x4 v[kGatherChunks];
+#pragma unroll
+  for (int u = 0; u < kGatherChunks; ++u) {
+    const int i = threadIdx.x + 256 * u, r = i / kRowChunks, ch = i - kRowChunks * r;
+    if (r < rows) v[u] = *reinterpret_cast<const u32x4*>(kv + s_src[r] + ch * 16);
+  }
+#pragma unroll
+  for (int u = 0; u < kGatherChunks; ++u) {
+    const int i = threadIdx.x + 256 * u, r = i / kRowChunks, ch = i - kRowChunks * r;
+    const int64_t dst = (int64_t)first * 64 + j0 + r;
+    if (r >= rows || dst < 0 || dst >= out_rows) continue;
     if (ch < 64)
-      *reinterpret_cast<u32x4*>(c_out + dst * c_row_bytes + ch * 16) = v;
+      *reinterpret_cast<u32x4*>(c_out + dst * c_row_bytes + ch * 16) = v[u];
     else
-      *reinterpret_cast<u32x4*>(rope_out + dst * rope_row_bytes + (ch - 64) * 16) = v;
+      *reinterpret_cast<u32x4*>(rope_out + dst * rope_row_bytes + (ch - 64) * 16) = v[u];
   }
 }
 
@@ -89,7 +103,7 @@ hipError_t launch_prefill_gather(const void* kv, int64_t kv_row_stride, int32_t 
                                  int64_t c_row_stride, void* rope_out, int64_t rope_row_stride, int64_t out_rows,
                                  int32_t* seg_pt, int64_t seg_pt_stride, hipStream_t stream) {
   if (batch == 0 || max_seg_pages == 0) return hipSuccess;
-  hipLaunchKernelGGL(prefill_gather_kernel, dim3(max_seg_pages, batch), dim3(256), 0, stream, (const char*)kv,
+  hipLaunchKernelGGL(prefill_gather_kernel, dim3(max_seg_pages * (64 / kGatherRows), batch), dim3(256), 0, stream, (const char*)kv,
                      kv_row_stride * 2, num_pages, log2_ps, page_table, pt_stride, seq_lens_k, seg_first,
                      (char*)c_out, c_row_stride * 2, (char*)rope_out, rope_row_stride * 2, out_rows, seg_pt,
                      seg_pt_stride);
