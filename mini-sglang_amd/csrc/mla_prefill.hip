@@ -185,19 +185,41 @@ __global__ __launch_bounds__(8 / QS * 64, 1) void mla_prefill_kernel(const Prefi
 
   // ---- work item: request b, query block qb, head group hg of HPC heads (groups fastest),
   // whose heads the CTA runs one after the other on the same request metadata and page-table
-  // sources; the last items (the latest query blocks, which see the most keys) are dispatched first
+  // sources. A request's last items (the latest query blocks, which see the most keys) are dispatched first,
+  // and of up to 64 requests the one with the most keys first: the long CTAs then do not run alone at the
+  // end (chunks of 531, 354 and 604 rows on prefixes of 2666, 197 and 296 keys, 64 heads: 119.3 us, 123.7 us in
+  // reverse request order)
   const int HG = (H + HPC - 1) / HPC;
-  auto items_of = [&](int r) __attribute__((always_inline)) {
-    return r < p.batch ? ((p.cu_seqlens_q[r + 1] - p.cu_seqlens_q[r] + kPrefillRows - 1) / kPrefillRows) * HG : 0;
-  };
-  int total = 0;
-  for (int c0 = 0; c0 < p.batch; c0 += 64) total += wave_sum(items_of(c0 + lane));
-  total = __builtin_amdgcn_readfirstlane(total);
-  const int item = total - 1 - (int)blockIdx.x;
   int b = -1, local = 0, q0 = 0, E = 0, L = 0;
-  if (item >= 0) {
+  int item = (int)blockIdx.x;
+  if (p.batch <= 64) {
+    const bool in = lane < p.batch;
+    const int lo = in ? p.cu_seqlens_q[lane] : 0, hi = in ? p.cu_seqlens_q[lane + 1] : 0, lk = in ? p.seq_lens_k[lane] : 0;
+    const int n = in ? ((hi - lo + kPrefillRows - 1) / kPrefillRows) * HG : 0;
+    int excl = 0;  // items of the requests before this lane's: longer ones, and as long ones of a lower index
+    for (int i = 0; i < p.batch; ++i) {
+      const int ni = __builtin_amdgcn_readlane(n, i), li = __builtin_amdgcn_readlane(lk, i);
+      if (li > lk || (li == lk && i < lane)) excl += ni;
+    }
+    const uint64_t hit = __ballot(in && item >= excl && item < excl + n);
+    if (hit != 0) {
+      const int fl = __builtin_ctzll(hit);
+      b = fl;
+      local = __builtin_amdgcn_readlane(n, fl) - 1 - (item - __builtin_amdgcn_readlane(excl, fl));
+      q0 = __builtin_amdgcn_readlane(lo, fl);
+      E = __builtin_amdgcn_readlane(hi, fl) - q0;
+      L = __builtin_amdgcn_readlane(lk, fl);
+    }
+  } else {
+    auto items_of = [&](int r) __attribute__((always_inline)) {
+      return r < p.batch ? ((p.cu_seqlens_q[r + 1] - p.cu_seqlens_q[r] + kPrefillRows - 1) / kPrefillRows) * HG : 0;
+    };
+    int total = 0;
+    for (int c0 = 0; c0 < p.batch; c0 += 64) total += wave_sum(items_of(c0 + lane));
+    total = __builtin_amdgcn_readfirstlane(total);
+    item = total - 1 - item;
     int acc = 0;
-    for (int c0 = 0; c0 < p.batch && b < 0; c0 += 64) {
+    for (int c0 = 0; item >= 0 && c0 < p.batch && b < 0; c0 += 64) {
       const int r = c0 + lane;
       const bool in = r < p.batch;
       // the request's query range and key count come with the scan (no second memory round trip)
