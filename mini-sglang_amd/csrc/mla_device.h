@@ -77,12 +77,14 @@ __device__ __forceinline__ void dma16_saddr_nt(const char* base, uint32_t voff, 
 __device__ __forceinline__ void dma16_vaddr(const char* addr, uint32_t lds_base) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(addr), "{m0}"(lds_base) : "memory");
 }
-// A 64-bit scalar base from a uniform vector value, for a DMA's address. A vector-ALU write of an
-// SGPR needs 5 wait states before a memory instruction reads it; readfirstlane and the nops are
-// volatile asm, so they stay in order with the DMA asm statements that follow.
+// A 64-bit scalar base from a uniform vector value, for a DMA's address. A lane read needs a wait state
+// after the vector-ALU write of its register (the compiler does not add it inside asm: without it the
+// low half was read before a v_lshl_add_u64 wrote it), and a vector-ALU write of an SGPR needs 5 before a
+// memory instruction reads it; readfirstlane and the nops are volatile asm, so they stay in order with the
+// DMA asm statements that follow.
 __device__ __forceinline__ const char* uniform_ptr(uint32_t lo, uint32_t hi) {
   uint32_t slo, shi;
-  asm volatile("v_readfirstlane_b32 %0, %2\n\tv_readfirstlane_b32 %1, %3\n\ts_nop 4"
+  asm volatile("s_nop 0\n\tv_readfirstlane_b32 %0, %2\n\tv_readfirstlane_b32 %1, %3\n\ts_nop 4"
                : "=s"(slo), "=s"(shi) : "v"(lo), "v"(hi));
   return reinterpret_cast<const char*>(((uint64_t)shi << 32) | slo);
 }
