@@ -73,7 +73,6 @@ struct MergeParams {
 // Chunked MLA prefill (non-absorbed): per-head K [.., 192] and V [.., 128] pools.
 constexpr int kPrefillQkDim = 192;
 constexpr int kPrefillVDim = 128;
-constexpr int kPrefillRows = 256;  // query rows per CTA (64 per wave)
 
 struct PrefillParams {
   const __bf16* q;  // [T, H, 192]
