@@ -15,7 +15,12 @@
 //        double-buffered P block in LDS
 //      output waves o = 0..3 (value dims 128o .. 128o+127, all 64 heads), one tile behind:
 //        O^T[128 dims x 64 heads] += V^T . P^T                 32 MFMAs, 16 transposing V reads
-//    Every K row is read from LDS by two waves, every V row by one. A SIMD holds one wave of each
+//    Every K row is read from LDS by two waves, every V row by one. Tiles are column blocks (mla_device.h):
+//    rows of 1152 bytes left the K reads 2-way bank conflicted, 12 of the 29 % of cycles the LDS was busy, and
+//    needed 9 source offsets per lane. Split step before -> after: 128 heads, 32 requests of 1k to 8k tokens
+//    79.6 -> 77.1 us (page size 1: 80.6 -> 76.3); 64 heads, 64 requests 74.3 -> 73.4 us (page size 1:
+//    78.0 -> 75.2); 8 requests of 1k to 8k tokens 18.6 -> 18.1; one of 1,500 tokens 11.35 -> 10.8 us.
+//    A SIMD holds one wave of each
 //    role, so one role's LDS and barrier waits are covered by the other's MFMAs. One barrier per step
 //    (two at a piece's first KV tile): step j scores tile j and accumulates tile j - 1; the output
 //    waves normalise and store a piece (bf16 output, or the bf16 partial of a split request) and
@@ -35,15 +40,11 @@ namespace {
 
 constexpr int kWWaves = 8;
 constexpr int kWAhead = 2;         // stream tiles in flight beyond the one being scored
-// A tile's 36 wave-wide DMA loads ("parts") are split between the roles: score wave r issues parts
-// r + 4k (k < kWScoreParts), output wave r parts 4 kWScoreParts + r + 4k (k < kWOutParts); a role
-// issues its parts after its step's work (instead of right after the step's barrier)
-// when its Late flag is set.
-constexpr int kWScoreParts = 0;
-constexpr int kWOutParts = 9;
-constexpr bool kWScoreLate = false;
-constexpr bool kWOutLate = false;
-static_assert(4 * (kWScoreParts + kWOutParts) == kTileDma, "every part of a tile is issued once");
+// Output wave r issues a tile's 9 loads of token octet r (one per column block), right after the step's barrier.
+// (Any of them on the score waves, at the step's start or after their work, measured 4 to 10 us more a launch: a
+// blocked issue stalls the score work, which is nearly critical too.)
+constexpr int kWParts = kTileBlocks;
+static_assert(4 * kWParts == kTileDma, "every load of a tile is issued once");
 constexpr int kWKPrefetch = 6;     // K operands in flight
 constexpr int kWVPrefetch = 4;     // V operand pairs in flight
 constexpr int kWMaxTiles = 2 * kMaxCtaBlocks;
@@ -67,8 +68,8 @@ struct WCursor {
 // step loops and spill.
 // kMode kPadded: 17 to 63 heads; query rows past the last head load the last head again and their outputs are
 // not written (the padding costs MFMAs, which the KV stream hides: 32 heads, 64 requests of 1k to 8k tokens,
-// 67.9 us against 78.1 us on the general kernel; 48 heads 70.7 against 82.5 us). kMode kGroups: more than 64 heads, in groups of 64 (the last one padded): CTA
-// blockIdx.x runs one group of one range, and the groups of a range are CTAs 8 apart, which the dispatcher
+// 67.9 us against 78.1 us on the general kernel; 48 heads 70.7 against 82.5 us).
+// kMode kGroups: more than 64 heads, in groups of 64 (the last one padded): CTA blockIdx.x runs one group of one range, and the groups of a range are CTAs 8 apart, which the dispatcher
 // puts on the same XCD at about the same time: the range's KV tiles come from HBM once and from that XCD's
 // L2 for the other groups (so they are loaded without the non-temporal hint). One launch per group, each
 // streaming the KV from HBM, took 80.8 us for 128 heads, 32 requests of 1k to 8k tokens; this takes 77.2 us
@@ -92,11 +93,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
     p.out = p0.out + (int64_t)h0 * p0.out_stride_h;
     if (p0.lse != nullptr) p.lse = p0.lse + h0;
   }
-  // a DMA load of KV rows: non-temporal where they are read once
-  auto dma_kv = [&](const char* base, uint32_t voff, uint32_t lds) __attribute__((always_inline)) {
-    if constexpr (kMode == kGroups) dma16_saddr(base, voff, lds);
-    else dma16_saddr_nt(base, voff, lds);
-  };
+  constexpr bool kNt = kMode != kGroups;  // KV loads are non-temporal where the rows are read once
   // first query row of query tile qt, and row t of it from there (rows past the last head: the last head)
   auto q_tile_row = [&](int qt) __attribute__((always_inline)) {
     return kMode == kExact ? 32 * qt : min(32 * qt, p.heads - 1);
@@ -138,16 +135,15 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
     const uint32_t lds_ring = (uint32_t)(uintptr_t)(MLA_LDS char*)smem;
 
     // ---- per-lane LDS read offsets (bytes within a tile)
-    const int xk = swz(c & 7);  // token 16 tb + c has the swizzle of token c
-    const int k_off_even = c * kRowBytes + ((g ^ xk) << 4);
-    const int k_off_odd = c * kRowBytes + (((4 + g) ^ xk) << 4);
-    int v_off[4];  // output wave `role`: value dims 128 role .. +128 start 256 role bytes into the row
+    const int xk = tswz(c);  // token 16 tb + c has the swizzle of token c
+    const int k_off_even = c * 128 + ((tperm(g) ^ xk) << 4);
+    const int k_off_odd = c * 128 + (((4 + tperm(g)) ^ xk) << 4);
+    int v_off[4];  // output wave `role`: value dims 128 role .. +128 are column blocks 2 role, 2 role + 1
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4)
-      v_off[q4] = (4 * g + (c >> 2)) * kRowBytes + 256 * role +
-                  ((2 * (q4 ^ (c >> 2)) + (((c & 3) >> 1) ^ (g & 1))) << 4) + ((c & 1) << 3);
-    // DMA: wave-wide load `part` of a tile covers slots 64 part + lane (token slot / 72, chunk slot % 72
-    // at its swizzled position); wave w issues parts w, w + 8, ... (score waves 5, output waves 4)
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const int t = 4 * g + (c >> 2);
+      v_off[q4] = 2 * role * kTileBlockBytes + t * 128 + (((2 * q4 + ((c & 3) >> 1)) ^ tswz(t)) << 4) + ((c & 1) << 3);
+    }
 
     // ---- stage the range: request bounds, then one page id per 32-token tile
     int rlast = (ke == 0 ? re - 1 : re);
@@ -159,22 +155,18 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
     // that they land while the range is staged (the staging's barriers wait on LDS only). If the
     // first piece turns out to be another request's, the stream issues its query tiles into the same
     // stages after these loads, and loads of one wave complete in order.
-    constexpr int kEarlyQueryDma = 2 * kWOutParts;
+    const int qrow_bytes = (int)(p.q_stride_h * 2);
+    auto issue_query = [&](int b, int qt, uint32_t stage) {  // this output wave's octet of query tile qt of request b
+      const char* qsrc = reinterpret_cast<const char*>(p.q) +
+                         ((int64_t)b * p.q_stride_b + (int64_t)q_tile_row(qt) * p.q_stride_h) * 2;
+      int ln;  // lane index from a volatile asm, so these offsets are computed here
+      asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+      const int t = octet_token(role, ln);
+      dma16_octet<false>(qsrc, q_row(t, qt) * qrow_bytes + octet_chunk(ln, t), stage + role * 1024);
+    };
     if (!scorer) {
-      const int qrow_bytes = (int)(p.q_stride_h * 2);
-#pragma unroll
-      for (int qt = 0; qt < 2; ++qt) {
-        const char* qsrc = reinterpret_cast<const char*>(p.q) +
-                           ((int64_t)rb * p.q_stride_b + (int64_t)q_tile_row(qt) * p.q_stride_h) * 2;
-#pragma unroll
-        for (int k = 0; k < kWOutParts; ++k) {
-          const int part = 4 * kWScoreParts + role + 4 * k;
-          const int s = part * 64 + lane;
-          const int t = (s * 7282) >> 19;  // s / 72
-          dma16_saddr(qsrc, q_row(t, qt) * qrow_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
-                      lds_ring + qt * kTileBytes + part * 1024);
-        }
-      }
+      issue_query(rb, 0, lds_ring);
+      issue_query(rb, 1, lds_ring + kTileBytes);
     }
     for (int r = threadIdx.x; r < nreq; r += kWWaves * 64) {
       const int b = rb + r;
@@ -256,59 +248,24 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
     // that role's state is live in its registers.
     auto run = [&](auto role_tag) {
     constexpr bool kScore = decltype(role_tag)::value;
-    constexpr int nparts = kScore ? kWScoreParts : kWOutParts;
-    const int part0 = kScore ? role : 4 * kWScoreParts + role;  // this wave's parts: part0 + 4k
-    uint32_t dma_voff[nparts > 0 ? nparts : 1];
-#pragma unroll
-    for (int k = 0; k < nparts; ++k) {
-      const int s = (part0 + 4 * k) * 64 + lane;
-      const int t = (s * 7282) >> 19;  // s / 72 for s < 2304
-      const int chunk_off = ((s - t * kRowChunks) ^ swz(t & 7)) << 4;
-      dma_voff[k] = kSmall ? (t << 16) | chunk_off : t * row_bytes + chunk_off;
-    }
+    constexpr int nparts = kScore ? 0 : kWParts;
+    const int dma_t = octet_token(role, lane);  // this lane's token of a tile, and its source offset there
+    const uint32_t dma_ch = octet_chunk(lane, dma_t);
     int iss_kv = 0;  // KV tiles issued (index into s_pid)
     // vector-memory operations this wave issued, and the count right after its parts of stream tile n
     // (kept for n % 4): tile n has landed once at most (ops - mark) operations are outstanding
-    int ops = kScore ? 0 : kEarlyQueryDma, mark0 = kScore ? 0 : kWOutParts, mark1 = ops, mark2 = 0, mark3 = 0;
+    int ops = 2 * nparts, mark0 = nparts, mark1 = ops, mark2 = 0, mark3 = 0;
     auto issue = [&](const WCursor& cur, int n) {  // this wave's DMA parts of stream tile n (at cur)
       const uint32_t stage = lds_ring + (n % kStages) * kTileBytes;
-      if (cur.q < 2) {  // query rows 32q .. +32 of request rb + r
-        const int qrow_bytes = (int)(p.q_stride_h * 2);
-        const char* qsrc = reinterpret_cast<const char*>(p.q) +
-                           ((int64_t)(rb + cur.r) * p.q_stride_b + (int64_t)q_tile_row(cur.q) * p.q_stride_h) * 2;
-        int ln;  // lane index from a volatile asm, so these offsets are computed here
-        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-#pragma unroll
-        for (int k = 0; k < nparts; ++k) {
-          const int s = (part0 + 4 * k) * 64 + ln;
-          const int t = (s * 7282) >> 19;
-          dma16_saddr(qsrc, q_row(t, cur.q) * qrow_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
-                      stage + (part0 + 4 * k) * 1024);
-        }
-      } else if constexpr (kSmall) {  // each lane's token row from the offset ring (clamped rows included)
-        const int ring = (n & 3) * 32;
-#pragma unroll
-        for (int k = 0; k < nparts; ++k)
-          dma_kv(kv, (uint32_t)s_pid[ring + (dma_voff[k] >> 16)] + (dma_voff[k] & 0xffff),
-                         stage + (part0 + 4 * k) * 1024);
+      if (cur.q < 2) {
+        issue_query(rb + cur.r, cur.q, stage);
+      } else if constexpr (kSmall) {  // the token's row from the offset ring (clamped rows included)
+        dma16_octet<kNt>(kv, (uint32_t)s_pid[(n & 3) * 32 + dma_t] + dma_ch, stage + role * 1024);
       } else {
         const int pid = __builtin_amdgcn_readfirstlane(s_pid[min(iss_kv++, kWMaxTiles - 1)]);
         const char* tsrc = kv + ((int64_t)pid * (ps_mask + 1) + (cur.t & ps_mask)) * row_bytes;
         const int tlim = cur.t1 - 1 - cur.t;  // loads clamp to the piece's last token
-        if (tlim >= kTile - 1) {
-#pragma unroll
-          for (int k = 0; k < nparts; ++k) dma_kv(tsrc, dma_voff[k], stage + (part0 + 4 * k) * 1024);
-        } else {
-          int ln;
-          asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
-#pragma unroll
-          for (int k = 0; k < nparts; ++k) {
-            const int s = (part0 + 4 * k) * 64 + ln;
-            const int t = (s * 7282) >> 19;
-            dma_kv(tsrc, min(t, tlim) * row_bytes + (((s - t * kRowChunks) ^ swz(t & 7)) << 4),
-                           stage + (part0 + 4 * k) * 1024);
-          }
-        }
+        dma16_octet<kNt>(tsrc, min(dma_t, tlim) * row_bytes + dma_ch, stage + role * 1024);
       }
       ops += nparts;
       const int m = n & 3;
@@ -467,8 +424,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
       }
       if (prev_kv && prev_end) attempt = 0;
 
-      constexpr bool kLate = kScore ? kWScoreLate : kWOutLate;
-      if (nparts > 0 && iss_valid && !kLate) {
+      if (nparts > 0 && iss_valid) {
         issue(iss, n_issued++);
         iss_valid = advance(iss);
       }
@@ -490,14 +446,14 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
             for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
               for (int ks = 0; ks < 18; ++ks) {
-                const int off = ((ks & 1) ? k_off_odd : k_off_even) + 128 * (ks >> 1) + 16 * hb * kRowBytes;
+                const int off = ((ks & 1) ? k_off_odd : k_off_even) + (ks >> 1) * kTileBlockBytes + 16 * hb * 128;
                 qf[hb][ks] = *reinterpret_cast<const MLA_LDS bf16x8*>(T + off);
               }
           }
         } else if (cur_kv) {
           // ---- S^T[16 tokens (half th) x 16 heads] for head blocks hb = 0, 1; two chains each
           auto kread = [&](int ks) {
-            const int off = ((ks & 1) ? k_off_odd : k_off_even) + 128 * (ks >> 1) + 16 * th * kRowBytes;
+            const int off = ((ks & 1) ? k_off_odd : k_off_even) + (ks >> 1) * kTileBlockBytes + 16 * th * 128;
             return *reinterpret_cast<const MLA_LDS bf16x8*>(T + off);
           };
           f32x4 sacc[2][2];
@@ -593,7 +549,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
         // blocks and all 4 head blocks
         const MLA_LDS char* T = (const MLA_LDS char*)smem + ((j - 1) % kStages) * kTileBytes;
         auto vread = [&](int db, int half) {
-          const int off = v_off[db & 3] + 128 * (db >> 2) + half * 16 * kRowBytes;
+          const int off = v_off[db & 3] + (db >> 2) * kTileBlockBytes + half * 16 * 128;
           return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((MLA_LDS bf16x4*)(T + off));
         };
         bf16x4 vlo[kWVPrefetch], vhi[kWVPrefetch];
@@ -680,10 +636,6 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
         }
       }
 
-      if (nparts > 0 && kLate && iss_valid) {  // this step's DMA after the work
-        issue(iss, n_issued++);
-        iss_valid = advance(iss);
-      }
       if constexpr (kSmall && kScore) if (role == 0) la_step();  // tile j + 3's offsets, tile j + 4 in flight
       // ---- advance: tile j becomes the previous tile
       prev_kv = cur_kv;

@@ -11,6 +11,22 @@ namespace mla {
 // position c ^ swz(t & 7).
 __device__ __forceinline__ int swz(int t7) { return ((t7 & 3) << 1) | ((t7 >> 2) & 1); }
 
+// Decode LDS tile of the streaming kernels: nine 128-byte column blocks, [block][32 tokens][128 B]; 16-byte chunk
+// ch of a block is stored at slot ch ^ tswz(token). Both operand reads are then bank-conflict free. A ds_read_b128
+// serves 16 lanes of 16 different tokens at a time, 8 of a 16-lane group and 8 of its neighbour; the groups read
+// chunks that differ by 2 (half 0 or 1 of a block: group g its chunk tperm(g); the same order for K and Q, so it only
+// permutes the dims of an MFMA k-step). A transposing read serves the chunk pairs of 8 tokens, which lie in different
+// slot pairs. Loads stay whole lines: a 1 KB DMA load is 8 tokens of a block, 128 bytes each, and a wave that loads
+// token octet o of every block needs one source offset per lane, plus 128 bytes a block.
+// (Rows of 1152 bytes with XOR-swizzled chunks left the K reads 2-way conflicted.)
+constexpr int kTileBlocks = kRowBytes / 128;
+constexpr int kTileBlockBytes = kTile * 128;
+__device__ __forceinline__ int tswz(int t) { return (((t >> 1) & 3) << 1) | ((t >> 3) & 1); }
+__device__ __forceinline__ int tperm(int g) { return ((g & 1) << 1) | (g >> 1); }
+// lane's token of octet o, and its source offset in the token's row (first block)
+__device__ __forceinline__ int octet_token(int o, int lane) { return 8 * o + (lane >> 3); }
+__device__ __forceinline__ uint32_t octet_chunk(int lane, int token) { return ((lane & 7) ^ tswz(token)) << 4; }
+
 // Combines a lane's value with lanes l ^ 16, l ^ 32 and l ^ 48 (the four lane groups; every lane gets the
 // result) by v_permlane16_swap / v_permlane32_swap: no LDS traffic and no LDS latency.
 template <typename F>
@@ -73,6 +89,24 @@ __device__ __forceinline__ void dma16_saddr(const char* base, uint32_t voff, uin
 // the lines that are reused.
 __device__ __forceinline__ void dma16_saddr_nt(const char* base, uint32_t voff, uint32_t lds_base) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(base), "{m0}"(lds_base) : "memory");
+}
+// Load of column block B (128 B bytes into the row, B KiB x 4 into the tile): the immediate offset is added to the
+// source and to the LDS address, so the LDS base gives it back.
+template <int B, bool kNt>
+__device__ __forceinline__ void dma16_block(const char* base, uint32_t voff, uint32_t lds_base) {
+  const uint32_t m0 = lds_base + B * (kTileBlockBytes - 128);
+  if constexpr (kNt)
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3 nt" ::"v"(voff), "s"(base), "{m0}"(m0), "n"(B * 128) : "memory");
+  else
+    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(voff), "s"(base), "{m0}"(m0), "n"(B * 128) : "memory");
+}
+// All blocks of a token octet: one wave's 9 loads of a tile.
+template <bool kNt, int B = 0>
+__device__ __forceinline__ void dma16_octet(const char* base, uint32_t voff, uint32_t lds_base) {
+  if constexpr (B < kTileBlocks) {
+    dma16_block<B, kNt>(base, voff, lds_base);
+    dma16_octet<kNt, B + 1>(base, voff, lds_base);
+  }
 }
 __device__ __forceinline__ void dma16_vaddr(const char* addr, uint32_t lds_base) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(addr), "{m0}"(lds_base) : "memory");
