@@ -13,8 +13,11 @@
 //    128 d .. +128 (16 transposing reads, 8 MFMAs).
 //  * the exponent reference is the piece's first-tile max and moves (O and l rescaled) only when a later
 //    score passes it by 2^64.
-// Measured (split step, 64 requests of 1k to 8k tokens, 363 MB, 8 heads): 64.1 us at page size 64 and
-// 64.5 us at page size 1 (5.7 TB/s), against 86.6 and 210.9 us of the general kernel, whose one wave runs a
+//  * tiles are column blocks (mla_device.h), with no bank conflicts and one source offset per lane for a
+//    wave's 9 loads of a tile: 67.7 -> 62.6 us against rows of 1152 bytes (page size 1: 64.1 -> 61.0; one
+//    request of 1,500 tokens: 7.1 -> 6.5 us), sizes as below.
+// Measured (split step, 64 requests of 1k to 8k tokens, 363 MB, 8 heads): 62.6 us at page size 64 and
+// 61.0 us at page size 1 (5.9 TB/s), against 86.6 and 210.9 us of the general kernel, whose one wave runs a
 // tile's MFMAs and 100 LDS reads as one serial chain and drains its ring at every piece. 17 heads and more
 // go to the warp-specialized kernel, padded to 64: a second head block here (eight waves) measured 72.0 us
 // against its 67.9 us at 32 heads.
@@ -24,10 +27,9 @@
 namespace mla {
 namespace {
 
-constexpr int kFWaves = 4;  // waves that load and compute; wave w issues DMA loads w, w + 4, ... of a tile
-constexpr int kFParts = kTileDma / kFWaves;  // loads of a KV tile per wave
-constexpr int kFQParts = 5;                  // loads per wave that hold the 16 query rows
-static_assert(kFWaves * kFQParts * 64 >= 16 * kRowChunks, "query rows");
+constexpr int kFWaves = 4;  // waves that load and compute; wave w issues a tile's loads of token octet w
+constexpr int kFParts = kTileBlocks;  // loads of a KV tile per wave, one per column block
+static_assert(kFWaves * kFParts == kTileDma, "every load of a tile is issued once");
 constexpr int kFAhead = 3;  // stream tiles in flight beyond the one being worked on
 constexpr int kFKPrefetch = 6;  // K operands in flight
 constexpr int kFVPrefetch = 4;  // V operand pairs in flight
@@ -68,8 +70,9 @@ struct RangeTables {
 // Fills the tables for the nreq (1..kMaxCtaRequests) requests of the range; every thread of the CTA calls it, and
 // it ends with a barrier (LDS only). A range inside one request, the usual case of a batch smaller than the
 // grid, needs no scan, and where the plan bounds it the page ids are requested before the request's length
-// is known (its blocks hold tokens of the request, so their entries exist): one memory round trip and one barrier where the general case takes two and three (split step of one 1,500-token
-// request: 7.35 -> 7.13 us; of 64 requests of 1k to 8k tokens: 68.5 -> 67.5 us).
+// is known (its blocks hold tokens of the request, so their entries exist): one memory round trip and one
+// barrier where the general case takes two and three (split step of one 1,500-token request: 7.35 -> 7.13 us;
+// of 64 requests of 1k to 8k tokens: 68.5 -> 67.5 us, when measured).
 template <int kThreads, bool kPages, int kPageCap>
 __device__ __forceinline__ void stage_range(const DecodeParams& p, int rb, int kb, int re, int ke, int nreq, int lane,
                                             int wave, const RangeTables& s) {
@@ -206,23 +209,17 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
     };
     const int lane = fresh_lane();
     const int g = lane >> 4, c = lane & 15;
-    // DMA slot s = 64 part + lane of a tile holds token s / 72, chunk (s % 72) ^ swz(token & 7)
-    auto slot_token = [&](int k, int ln) { return (((wave + kFWaves * k) * 64 + ln) * 7282) >> 19; };  // s / 72
-    auto slot_chunk16 = [&](int k, int ln, int t) {
-      return (((wave + kFWaves * k) * 64 + ln - t * kRowChunks) ^ swz(t & 7)) << 4;
-    };
+    // the 16 query rows are octets 0 and 1 of a tile: waves 0 and 1 load them
+    const int nq = wave < 2 ? kFParts : 0;
     auto issue_query = [&](int b, uint32_t stage) {  // rows past the last head load the last head
+      if (wave >= 2) return;
       const char* src = reinterpret_cast<const char*>(p.q) + (int64_t)b * p.q_stride_b * 2;
-      const int ln = fresh_lane();
-#pragma unroll
-      for (int k = 0; k < kFQParts; ++k) {
-        const int t = slot_token(k, ln);
-        dma16_saddr(src, min(t, H - 1) * qrow_bytes + slot_chunk16(k, ln, t), stage + (wave + kFWaves * k) * 1024);
-      }
+      const int ln = fresh_lane(), t = octet_token(wave, ln);
+      dma16_octet<false>(src, min(t, H - 1) * qrow_bytes + octet_chunk(ln, t), stage + wave * 1024);
     };
     // The first piece is request rb's unless its part of the range is empty (only for an empty request): its
     // queries land in ring stage 0 while the range is staged (the staging's barriers wait on LDS only).
-    if (!kSmall || wave < kFWaves) issue_query(rb, lds_ring);
+    issue_query(rb, lds_ring);
 
     stage_range<kThreads, !kSmall, kFMaxTiles>(p, rb, kb, re, ke, nreq, lane, wave,
                                                RangeTables{s_t0, s_t1, s_tbase, s_np, s_slot0, s_pid});
@@ -295,55 +292,35 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
 
     // ---- per-lane LDS read offsets (bytes within a tile)
     const int th = wave & 1, kh = wave >> 1;
-    const int xk = swz(c & 7);  // token 16 tb + c has the swizzle of token c
-    const int k_even = c * kRowBytes + ((g ^ xk) << 4), k_odd = c * kRowBytes + (((4 + g) ^ xk) << 4);
-    // operand i of this wave's dim half is k-step 9 kh + i (32 dims each)
-    const int k_a = kh ? k_odd + 4 * 128 : k_even, k_b = kh ? k_even + 5 * 128 : k_odd;
-    int v_off[4];
+    const int xk = tswz(c);  // token 16 tb + c has the swizzle of token c
+    const int k_lo = c * 128 + ((tperm(g) ^ xk) << 4), k_hi = c * 128 + (((4 + tperm(g)) ^ xk) << 4);
+    // operand i of this wave's dim half is k-step 9 kh + i (half a column block each)
+    const int k_a = kh ? k_hi + 4 * kTileBlockBytes : k_lo, k_b = kh ? k_lo + 5 * kTileBlockBytes : k_hi;
+    int v_off[4];  // value dims 128 wave .. +128 are column blocks 2 wave, 2 wave + 1
 #pragma unroll
-    for (int q4 = 0; q4 < 4; ++q4)
-      v_off[q4] = (4 * g + (c >> 2)) * kRowBytes + 256 * wave +
-                  ((2 * (q4 ^ (c >> 2)) + (((c & 3) >> 1) ^ (g & 1))) << 4) + ((c & 1) << 3);
-
-    uint32_t dma_voff[kFParts];
-#pragma unroll
-    for (int k = 0; k < kFParts; ++k) {
-      const int t = slot_token(k, lane), ch = slot_chunk16(k, lane, t);
-      dma_voff[k] = kSmall ? (uint32_t)((t << 16) | ch) : (uint32_t)(t * row_bytes + ch);
+    for (int q4 = 0; q4 < 4; ++q4) {
+      const int t = 4 * g + (c >> 2);
+      v_off[q4] = 2 * wave * kTileBlockBytes + t * 128 + (((2 * q4 + ((c & 3) >> 1)) ^ tswz(t)) << 4) + ((c & 1) << 3);
     }
+    const int dma_t = octet_token(wave, lane);  // this lane's token of a tile, and its source offset there
+    const uint32_t dma_ch = octet_chunk(lane, dma_t);
     int iss_kv = 0;  // KV tiles issued (index into s_pid)
     // vector-memory operations this wave issued, and the count right after its loads of stream tile n
     // (kept for n % 4): tile n has landed once at most (ops - mark) operations are outstanding
-    int ops = kFQParts, mark0 = kFQParts, mark1 = 0, mark2 = 0, mark3 = 0;
+    int ops = nq, mark0 = nq, mark1 = 0, mark2 = 0, mark3 = 0;
     auto issue = [&](const FCursor& cur, int n) {  // this wave's loads of stream tile n (at cur)
       const uint32_t stage = lds_ring + (n % kStages) * kTileBytes;
       if (cur.q == 0) {
         issue_query(rb + cur.r, stage);
-        ops += kFQParts;
+        ops += nq;
       } else {
-        if constexpr (kSmall) {
-#pragma unroll
-          for (int k = 0; k < kFParts; ++k) {
-            dma16_saddr_nt(kv, (uint32_t)s_pid[(n & 3) * kTile + (dma_voff[k] >> 16)] + (dma_voff[k] & 0xffff),
-                           stage + (wave + kFWaves * k) * 1024);
-          }
+        if constexpr (kSmall) {  // the token's row from the offset ring (clamped rows included)
+          dma16_octet<true>(kv, (uint32_t)s_pid[(n & 3) * kTile + dma_t] + dma_ch, stage + wave * 1024);
         } else {
-          const int tlim = cur.t1 - 1 - cur.t;  // loads clamp to the piece's last token
           const int pid = __builtin_amdgcn_readfirstlane(s_pid[min(iss_kv++, kFMaxTiles - 1)]);
           const char* src = kv + ((int64_t)pid * (ps_mask + 1) + (cur.t & ps_mask)) * row_bytes;
-          if (tlim >= kTile - 1) {
-#pragma unroll
-            for (int k = 0; k < kFParts; ++k) {
-              dma16_saddr_nt(src, dma_voff[k], stage + (wave + kFWaves * k) * 1024);
-            }
-          } else {
-            const int ln = fresh_lane();
-#pragma unroll
-            for (int k = 0; k < kFParts; ++k) {
-              const int t = slot_token(k, ln);
-              dma16_saddr_nt(src, min(t, tlim) * row_bytes + slot_chunk16(k, ln, t), stage + (wave + kFWaves * k) * 1024);
-            }
-          }
+          const int tlim = cur.t1 - 1 - cur.t;  // loads clamp to the piece's last token
+          dma16_octet<true>(src, min(dma_t, tlim) * row_bytes + dma_ch, stage + wave * 1024);
         }
         ops += kFParts;
       }
@@ -389,12 +366,12 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
       if (cs.q == 0) {  // a piece starts: this wave's dim half of the query rows
 #pragma unroll
         for (int i = 0; i < 9; ++i)
-          qf[i] = *reinterpret_cast<const MLA_LDS bf16x8*>(T + ((i & 1) ? k_b : k_a) + 128 * (i >> 1));
+          qf[i] = *reinterpret_cast<const MLA_LDS bf16x8*>(T + ((i & 1) ? k_b : k_a) + kTileBlockBytes * (i >> 1));
       } else {
         // ---- partial S^T[16 tokens (half th) x 16 heads] over dims 288 kh .. +288
-        const MLA_LDS char* K = T + th * (16 * kRowBytes);
+        const MLA_LDS char* K = T + th * (16 * 128);
         auto kread = [&](int i) {
-          return *reinterpret_cast<const MLA_LDS bf16x8*>(K + ((i & 1) ? k_b : k_a) + 128 * (i >> 1));
+          return *reinterpret_cast<const MLA_LDS bf16x8*>(K + ((i & 1) ? k_b : k_a) + kTileBlockBytes * (i >> 1));
         };
         f32x4 sacc[2];
         sacc[0] = sacc[1] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -415,7 +392,7 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
         for (int t = 0; t < 2; ++t) sv[t] = s_s[0][t][lane] + s_s[1][t][lane];
         // the V^T operands do not depend on the softmax: read the first ones now
         auto vread = [&](int db, int half) {
-          const int off = v_off[db & 3] + 128 * (db >> 2) + half * 16 * kRowBytes;
+          const int off = v_off[db & 3] + kTileBlockBytes * (db >> 2) + half * 16 * 128;
           return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((MLA_LDS bf16x4*)(T + off));
         };
         bf16x4 vlo[kFVPrefetch], vhi[kFVPrefetch];
