@@ -355,7 +355,7 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
     for (int j = 0;; ++j) {
       {  // tile j lands: wait for this wave's loads of it, then the whole CTA's; stage (j - 1) % 4 is free
         const int m = j & 3;
-        wait_vmcnt_dyn(ops - (m == 0 ? mark0 : m == 1 ? mark1 : m == 2 ? mark2 : mark3));
+        wait_vmcnt_dyn<(kFAhead - 1) * kFParts>(ops - (m == 0 ? mark0 : m == 1 ? mark1 : m == 2 ? mark2 : mark3));
       }
       barrier_lds();
       if (iss_valid) {

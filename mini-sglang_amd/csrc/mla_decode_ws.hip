@@ -40,6 +40,7 @@ namespace {
 
 constexpr int kWWaves = 8;
 constexpr int kWAhead = 2;         // stream tiles in flight beyond the one being scored
+static_assert(kWAhead == 2, "two marks beyond the step's own");
 // Output wave r issues a tile's 9 loads of token octet r (one per column block), right after the step's barrier.
 // (Any of them on the score waves, at the step's start or after their work, measured 4 to 10 us more a launch: a
 // blocked issue stalls the score work, which is nearly critical too.)
@@ -252,9 +253,13 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
     const int dma_t = octet_token(role, lane);  // this lane's token of a tile, and its source offset there
     const uint32_t dma_ch = octet_chunk(lane, dma_t);
     int iss_kv = 0;  // KV tiles issued (index into s_pid)
-    // vector-memory operations this wave issued, and the count right after its parts of stream tile n
-    // (kept for n % 4): tile n has landed once at most (ops - mark) operations are outstanding
-    int ops = 2 * nparts, mark0 = nparts, mark1 = ops, mark2 = 0, mark3 = 0;
+    // vector-memory operations this wave issued, and the count right after its loads of the stream tiles of this
+    // step and the next two: a tile has landed once at most (ops - mark) operations are outstanding
+    int ops = 2 * nparts, mark0 = nparts, mark1 = ops, mark2 = 0;
+    int pid_v = 0;  // !kSmall: page id of KV tile iss_kv, read a step ahead of its use
+    auto fetch_pid = [&]() {
+      if constexpr (!kSmall) pid_v = s_pid[min(iss_kv, kWMaxTiles - 1)];
+    };
     auto issue = [&](const WCursor& cur, int n) {  // this wave's DMA parts of stream tile n (at cur)
       const uint32_t stage = lds_ring + (n % kStages) * kTileBytes;
       if (cur.q < 2) {
@@ -262,17 +267,14 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
       } else if constexpr (kSmall) {  // the token's row from the offset ring (clamped rows included)
         dma16_octet<kNt>(kv, (uint32_t)s_pid[(n & 3) * 32 + dma_t] + dma_ch, stage + role * 1024);
       } else {
-        const int pid = __builtin_amdgcn_readfirstlane(s_pid[min(iss_kv++, kWMaxTiles - 1)]);
+        const int pid = __builtin_amdgcn_readfirstlane(pid_v);
+        ++iss_kv;
         const char* tsrc = kv + ((int64_t)pid * (ps_mask + 1) + (cur.t & ps_mask)) * row_bytes;
         const int tlim = cur.t1 - 1 - cur.t;  // loads clamp to the piece's last token
         dma16_octet<kNt>(tsrc, min(dma_t, tlim) * row_bytes + dma_ch, stage + role * 1024);
       }
       ops += nparts;
-      const int m = n & 3;
-      mark0 = m == 0 ? ops : mark0;
-      mark1 = m == 1 ? ops : mark1;
-      mark2 = m == 2 ? ops : mark2;
-      mark3 = m == 3 ? ops : mark3;
+      fetch_pid();
     };
 
     WCursor cs;  // the tile scored at this step
@@ -296,8 +298,10 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
     }
     auto prologue = [&](const int from) {
       if constexpr (nparts == 0) return;  // a role without DMA parts keeps no issue cursor
+      fetch_pid();
       for (int s = from; s < kWAhead && iss_valid; ++s) {
         issue(iss, n_issued++);
+        (s == 0 ? mark0 : mark1) = ops;
         iss_valid = advance(iss);
       }
     };
@@ -376,10 +380,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
 
     for (int j = 0;;) {
       // ---- step j: tile j (cs) lands; wait for this wave's DMA parts of it, then the whole CTA's
-      if (j < n_issued) {
-        const int m = j & 3;
-        wait_vmcnt_dyn(ops - (m == 0 ? mark0 : m == 1 ? mark1 : m == 2 ? mark2 : mark3));
-      }
+      if (nparts > 0 && s_valid) wait_vmcnt_dyn<(kWAhead - 1) * kWParts>(ops - mark0);
       barrier_lds();
 
       if (prev_kv && prev_end && attempt == 0 && (s_flag[0] | s_flag[1] | s_flag[2] | s_flag[3]) != 0) {
@@ -426,6 +427,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
 
       if (nparts > 0 && iss_valid) {
         issue(iss, n_issued++);
+        mark2 = ops;
         iss_valid = advance(iss);
       }
 
@@ -646,6 +648,8 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
         first_kv = cur_end;  // the next KV tile starts a piece
       }
       if (s_valid) s_valid = advance(cs);
+      mark0 = mark1;
+      mark1 = mark2;
       ++j;
       if (!s_valid && !prev_kv) break;
     }

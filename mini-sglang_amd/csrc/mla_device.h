@@ -154,23 +154,32 @@ __device__ __forceinline__ void sload_i32x4(const int32_t* ptr, int& a, int& b, 
   d = v[3];
 }
 
-// Binary tree of scalar branches over the wait count (6 compares for 0..63).
+// Binary tree of scalar branches over wait counts 8 Lo, 8 (Lo + 1), ... 8 Hi.
 template <int Lo, int Hi>
 __device__ __forceinline__ void wait_vmcnt_tree(int n) {
   if constexpr (Lo == Hi) {
-    wait_vmcnt<Lo>();
+    wait_vmcnt<8 * Lo>();
   } else {
     constexpr int Mid = (Lo + Hi) / 2;
-    if (n <= Mid) wait_vmcnt_tree<Lo, Mid>(n);
+    if (n < 8 * (Mid + 1)) wait_vmcnt_tree<Lo, Mid>(n);
     else wait_vmcnt_tree<Mid + 1, Hi>(n);
   }
 }
 
-// wait_vmcnt with a run-time count, clamped to the counter range. The count is
-// made wave-uniform first so that the selection compiles to scalar branches.
+// wait_vmcnt with a run-time count (clamped to the counter range, made wave-uniform so that the selection
+// compiles to scalar branches). kUsual, the count of a loop's steady state, is tested first, and other counts
+// (after a piece's stores, at the stream's end) wait for a multiple of 8, at most 7 operations more than they need:
+// a tree of all 64 counts took about 550 cycles of a decode step's 3200 (split step of 64 requests of 1k to 8k
+// tokens, 8 heads: 62.2 -> 58.9 us; 64 heads, with its marks and page ids kept a step ahead: 73.7 -> 71.1 us;
+// 8 requests of 32k to 128k tokens, 64 heads: 158.5 -> 147.5 us).
+template <int kUsual>
 __device__ __forceinline__ void wait_vmcnt_dyn(int n) {
-  n = __builtin_amdgcn_readfirstlane(n > 63 ? 63 : (n < 0 ? 0 : n));
-  wait_vmcnt_tree<0, 63>(n);
+  n = __builtin_amdgcn_readfirstlane(n);
+  if (n == kUsual) {
+    wait_vmcnt<kUsual>();
+    return;
+  }
+  wait_vmcnt_tree<0, 7>(n > 63 ? 63 : (n < 0 ? 0 : n));
 }
 
 }  // namespace mla
