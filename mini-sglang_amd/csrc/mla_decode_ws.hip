@@ -33,6 +33,7 @@
 #include <type_traits>
 
 #include "mla_common.h"
+#include "mla_decode_stage.h"
 #include "mla_device.h"
 
 namespace mla {
@@ -169,61 +170,8 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
       issue_query(rb, 0, lds_ring);
       issue_query(rb, 1, lds_ring + kTileBytes);
     }
-    for (int r = threadIdx.x; r < nreq; r += kWWaves * 64) {
-      const int b = rb + r;
-      const int L = p.seq_lens[b];
-      const int t0 = (r == 0) ? kb * kPlanBlock : 0;
-      const int t1 = max(t0, (b == re) ? min(ke * kPlanBlock, L) : L);
-      s_t0[r] = t0;
-      s_t1[r] = t1;
-      s_tbase[r + 1] = (t1 - t0 + kTile - 1) / kTile;
-      const int first = p.plan[4 * p.num_ctas + 3 * b + 0];
-      s_np[r] = p.plan[4 * p.num_ctas + 3 * b + 1];
-      s_slot0[r] = p.plan[4 * p.num_ctas + 3 * b + 2] - first;
-    }
-    barrier_lds();
-    if (wave == 0) {  // exclusive prefix of tile counts (64-wide scans)
-      int carry = 0;
-      for (int c0 = 0; c0 < nreq; c0 += 64) {
-        const int r = c0 + lane;
-        int v = r < nreq ? s_tbase[r + 1] : 0;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-          const int u = __shfl_up(v, o);
-          if (lane >= o) v += u;
-        }
-        if (r < nreq) s_tbase[r + 1] = carry + v;
-        carry += __shfl(v, 63);
-      }
-      if (lane == 0) s_tbase[0] = 0;
-    }
-    barrier_lds();
-    const int ntiles_cta = min(s_tbase[nreq], kWMaxTiles);
-    if constexpr (!kSmall) {
-      constexpr int kPer = kWMaxTiles / (kWWaves * 64);
-      int pid[kPer];
-#pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        const int k = threadIdx.x + kWWaves * 64 * u;
-        pid[u] = 0;
-        if (k < ntiles_cta) {
-          int lo = 0, hi = nreq - 1;  // last request whose first tile is <= k
-          while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (s_tbase[mid] <= k) lo = mid;
-            else hi = mid - 1;
-          }
-          const int t = s_t0[lo] + kTile * (k - s_tbase[lo]);
-          pid[u] = p.page_table[(int64_t)(rb + lo) * p.pt_stride + (t >> p.log2_ps)];
-        }
-      }
-#pragma unroll
-      for (int u = 0; u < kPer; ++u) {
-        const int k = threadIdx.x + kWWaves * 64 * u;
-        if (k < ntiles_cta) s_pid[k] = min(max(pid[u], 0), p.num_pages - 1);
-      }
-    }
-    barrier_lds();
+    stage_range<kWWaves * 64, !kSmall, kWMaxTiles>(p, rb, kb, re, ke, nreq, lane, wave,
+                                                   RangeTables{s_t0, s_t1, s_tbase, s_np, s_slot0, s_pid});
 
     // ---- stream cursors over (request, tile); all values wave-uniform
     auto seek = [&](WCursor& cur, int r) -> bool {  // first non-empty piece at or after request rb + r
