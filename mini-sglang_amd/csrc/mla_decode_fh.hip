@@ -36,7 +36,7 @@ constexpr int kFKPrefetch = 6;  // K operands in flight
 constexpr int kFVPrefetch = 4;  // V operand pairs in flight
 constexpr int kFMaxTiles = 2 * kMaxCtaBlocks;
 constexpr float kFRescaleLog2 = 64.0f;
-static_assert(kFAhead == kStages - 1, "a tile is issued into the stage of the tile just finished");
+static_assert(kFAhead == kStages - 1 && kFAhead == 3, "a tile is issued into the stage of the tile just finished");
 
 struct FCursor {
   int r, t, t0, t1, q;  // request rb + r, piece [t0, t1); q == 0: query tile, q == 1: KV tile at token t
@@ -180,9 +180,10 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
     const int dma_t = octet_token(wave, lane);  // this lane's token of a tile, and its source offset there
     const uint32_t dma_ch = octet_chunk(lane, dma_t);
     int iss_kv = 0;  // KV tiles issued (index into s_pid)
-    // vector-memory operations this wave issued, and the count right after its loads of stream tile n
-    // (kept for n % 4): tile n has landed once at most (ops - mark) operations are outstanding
+    // vector-memory operations this wave issued, and the count right after its loads of the stream tiles of this
+    // step and the next three: a tile has landed once at most (ops - mark) operations are outstanding
     int ops = nq, mark0 = nq, mark1 = 0, mark2 = 0, mark3 = 0;
+    int pid_v = kSmall ? 0 : s_pid[0];  // page id of KV tile iss_kv, read a step ahead of its use
     auto issue = [&](const FCursor& cur, int n) {  // this wave's loads of stream tile n (at cur)
       const uint32_t stage = lds_ring + (n % kStages) * kTileBytes;
       if (cur.q == 0) {
@@ -192,18 +193,14 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
         if constexpr (kSmall) {  // the token's row from the offset ring (clamped rows included)
           dma16_octet<true>(kv, (uint32_t)s_pid[(n & 3) * kTile + dma_t] + dma_ch, stage + wave * 1024);
         } else {
-          const int pid = __builtin_amdgcn_readfirstlane(s_pid[min(iss_kv++, kFMaxTiles - 1)]);
+          const int pid = __builtin_amdgcn_readfirstlane(pid_v);
+          pid_v = s_pid[min(++iss_kv, kFMaxTiles - 1)];
           const char* src = kv + ((int64_t)pid * (ps_mask + 1) + (cur.t & ps_mask)) * row_bytes;
           const int tlim = cur.t1 - 1 - cur.t;  // loads clamp to the piece's last token
           dma16_octet<true>(src, min(dma_t, tlim) * row_bytes + dma_ch, stage + wave * 1024);
         }
         ops += kFParts;
       }
-      const int m = n & 3;
-      mark0 = m == 0 ? ops : mark0;
-      mark1 = m == 1 ? ops : mark1;
-      mark2 = m == 2 ? ops : mark2;
-      mark3 = m == 3 ? ops : mark3;
     };
 
     if constexpr (kSmall) barrier_lds();  // the first tiles' row offsets are written
@@ -217,7 +214,9 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
       wait_vmcnt<0>();
     }
     while (n_issued < kFAhead && iss_valid) {
-      issue(iss, n_issued++);
+      issue(iss, n_issued);
+      (n_issued == 0 ? mark0 : n_issued == 1 ? mark1 : mark2) = ops;
+      ++n_issued;
       iss_valid = advance(iss);
     }
 
@@ -228,13 +227,12 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
     for (int db = 0; db < 8; ++db) O[db] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     for (int j = 0;; ++j) {
-      {  // tile j lands: wait for this wave's loads of it, then the whole CTA's; stage (j - 1) % 4 is free
-        const int m = j & 3;
-        wait_vmcnt_dyn<(kFAhead - 1) * kFParts>(ops - (m == 0 ? mark0 : m == 1 ? mark1 : m == 2 ? mark2 : mark3));
-      }
+      // tile j lands: wait for this wave's loads of it, then the whole CTA's; stage (j - 1) % 4 is free
+      wait_vmcnt_dyn<(kFAhead - 1) * kFParts>(ops - mark0);
       barrier_lds();
       if (iss_valid) {
         issue(iss, n_issued++);
+        mark3 = ops;
         iss_valid = advance(iss);
       }
       const MLA_LDS char* T = (const MLA_LDS char*)smem + (j % kStages) * kTileBytes;
@@ -369,6 +367,9 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
           for (int db = 0; db < 8; ++db) O[db] = f32x4{0.f, 0.f, 0.f, 0.f};
         }
       }
+      mark0 = mark1;
+      mark1 = mark2;
+      mark2 = mark3;
       if (!advance(cs)) break;
     }
     return true;
