@@ -16,11 +16,11 @@
 //  * tiles are column blocks (mla_device.h), with no bank conflicts and one source offset per lane for a
 //    wave's 9 loads of a tile: 67.7 -> 62.6 us against rows of 1152 bytes (page size 1: 64.1 -> 61.0; one
 //    request of 1,500 tokens: 7.1 -> 6.5 us), sizes as below.
-// Measured (split step, 64 requests of 1k to 8k tokens, 363 MB, 8 heads): 62.6 us at page size 64 and
-// 61.0 us at page size 1 (5.9 TB/s), against 86.6 and 210.9 us of the general kernel, whose one wave runs a
+// Measured (split step, 64 requests of 1k to 8k tokens, 363 MB, 8 heads): 58.7 us at page size 64 (6.2
+// TB/s) and 60.4 us at page size 1, against 86.6 and 210.9 us of the general kernel, whose one wave runs a
 // tile's MFMAs and 100 LDS reads as one serial chain and drains its ring at every piece. 17 heads and more
 // go to the warp-specialized kernel, padded to 64: a second head block here (eight waves) measured 72.0 us
-// against its 67.9 us at 32 heads.
+// against its 67.9 us at 32 heads (both before the tile layout changed).
 #include "mla_common.h"
 #include "mla_decode_stage.h"
 #include "mla_device.h"

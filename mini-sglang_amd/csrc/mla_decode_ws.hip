@@ -28,8 +28,10 @@
 //  * No accumulator rescaling: exponents are taken against the piece's first-tile max; a piece whose
 //    later scores exceed it by 2^64 is rerun with its exact max (the vote is taken at the step after
 //    the piece's last tile, before any wave touches the next tile).
-//  * Barriers wait on LDS only; each wave counts its own DMA loads and output stores and waits with
-//    an exact vmcnt.
+//  * Barriers wait on LDS only; each wave counts its own DMA loads and output stores and waits for
+//    a tile's loads by that count (wait_vmcnt_dyn).
+// Bound: the output waves' chain (about 2,800 cycles a tile: 1,000 to issue their nine loads, 1,330 of operand
+// reads and MFMAs), just above the tile's HBM time (2,700 cycles).
 #include <type_traits>
 
 #include "mla_common.h"
@@ -42,7 +44,7 @@ namespace {
 constexpr int kWWaves = 8;
 constexpr int kWAhead = 2;         // stream tiles in flight beyond the one being scored
 static_assert(kWAhead == 2, "two marks beyond the step's own");
-// Output wave r issues a tile's 9 loads of token octet r (one per column block), right after the step's barrier.
+// Output wave r issues a tile's 9 loads of token octet r (one per column block) at the step's start.
 // (Any of them on the score waves, at the step's start or after their work, measured 4 to 10 us more a launch: a
 // blocked issue stalls the score work, which is nearly critical too.)
 constexpr int kWParts = kTileBlocks;
@@ -74,8 +76,8 @@ struct WCursor {
 // kMode kGroups: more than 64 heads, in groups of 64 (the last one padded): CTA blockIdx.x runs one group of one range, and the groups of a range are CTAs 8 apart, which the dispatcher
 // puts on the same XCD at about the same time: the range's KV tiles come from HBM once and from that XCD's
 // L2 for the other groups (so they are loaded without the non-temporal hint). One launch per group, each
-// streaming the KV from HBM, took 80.8 us for 128 heads, 32 requests of 1k to 8k tokens; this takes 77.2 us
-// (the step is then bound by the waves' own chain of loads, MFMAs and barriers, no longer by HBM).
+// streaming the KV from HBM, took 80.8 us for 128 heads, 32 requests of 1k to 8k tokens, where this took 77.2 us
+// (and 66 us with the tile layout and waits of today; HBM no longer bounds it).
 enum WMode { kExact, kPadded, kGroups };
 
 template <bool kSmall, bool kLoop, WMode kMode>
@@ -373,11 +375,17 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
       }
       if (prev_kv && prev_end) attempt = 0;
 
-      if (nparts > 0 && iss_valid) {
-        issue(iss, n_issued++);
-        mark2 = ops;
-        iss_valid = advance(iss);
-      }
+      auto issue_next = [&]() __attribute__((always_inline)) {
+        if (nparts > 0 && iss_valid) {
+          issue(iss, n_issued++);
+          mark2 = ops;
+          iss_valid = advance(iss);
+        }
+      };
+      // An output step requests its first LDS operands before it issues, so that they arrive meanwhile (split step,
+      // 8 requests of 32k to 128k tokens: 147.3 -> 144.7 us; 64 of 1k to 8k: 69.7 -> 69.2). With small pages the
+      // issue itself begins with an LDS read, and comes first (1.5 % slower after the operands).
+      if (kSmall || !prev_kv) issue_next();
 
       const bool cur_kv = s_valid && cs.q == 2;
       const bool cur_end = cur_kv && cs.t + kTile >= cs.t1;
@@ -511,6 +519,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
         bf16x8 pb[4];
 #pragma unroll
         for (int hq = 0; hq < 4; ++hq) pb[hq] = __builtin_bit_cast(bf16x8, s_p[(j - 1) & 1][hq][lane]);
+        if constexpr (!kSmall) issue_next();
 #pragma unroll
         for (int db = 0; db < 8; ++db) {
           const bf16x8 a =
