@@ -85,13 +85,9 @@ __device__ __forceinline__ void wait_vmcnt() {
 __device__ __forceinline__ void dma16_saddr(const char* base, uint32_t voff, uint32_t lds_base) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "{m0}"(lds_base) : "memory");
 }
-// The same with the non-temporal hint: for data read once (streamed KV rows), so the caches keep
-// the lines that are reused.
-__device__ __forceinline__ void dma16_saddr_nt(const char* base, uint32_t voff, uint32_t lds_base) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 nt" ::"v"(voff), "s"(base), "{m0}"(lds_base) : "memory");
-}
 // Load of column block B (128 B bytes into the row, B KiB x 4 into the tile): the immediate offset is added to the
-// source and to the LDS address, so the LDS base gives it back.
+// source and to the LDS address, so the LDS base gives it back. kNt: the non-temporal hint, for data read once
+// (streamed KV rows), so the caches keep the lines that are reused.
 template <int B, bool kNt>
 __device__ __forceinline__ void dma16_block(const char* base, uint32_t voff, uint32_t lds_base) {
   const uint32_t m0 = lds_base + B * (kTileBlockBytes - 128);
