@@ -34,10 +34,9 @@ struct RangeTables {
 
 // Fills the tables for the nreq (1..kMaxCtaRequests) requests of the range; every thread of the CTA calls it, and
 // it ends with a barrier (LDS only). A range inside one request, the usual case of a batch smaller than the
-// grid, needs no scan, and where the plan bounds it the page ids are requested before the request's length
-// is known (its blocks hold tokens of the request, so their entries exist): one memory round trip and one
-// barrier where the general case takes two and three (split step of one 1,500-token request, 8 heads: 7.35 ->
-// 7.13 us, 64 heads: 9.95 -> 9.51, 128 heads: 10.4 -> 9.9; 8 requests of 1k to 8k tokens, 64 heads: 17.4 -> 16.8).
+// grid, needs no scan and one barrier where the general case takes three. The page ids are read once the
+// request's length is known: what bounds the columns of a row that exist is its length alone, not the plan
+// (made for another step's lengths, perhaps) nor the table's row stride (1 for a one-row table's transpose).
 template <int kThreads, bool kPages, int kPageCap>
 __device__ __forceinline__ void stage_range(const DecodeParams& p, int rb, int kb, int re, int ke, int nreq, int lane,
                                             int wave, const RangeTables& s) {
@@ -50,16 +49,14 @@ __device__ __forceinline__ void stage_range(const DecodeParams& p, int rb, int k
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
       const int t = t0 + kTile * (tid + kThreads * u);
-      pid[u] = t < t1 ? row[min((int64_t)(t >> p.log2_ps), p.pt_stride - 1)] : 0;
+      pid[u] = t < t1 ? row[t >> p.log2_ps] : 0;
     }
   };
   if (nreq == 1) {
     const int t0 = kb * kPlanBlock;
-    const bool bounded = re == rb;  // the range ends inside request rb: its blocks hold tokens
-    if constexpr (kPages) if (bounded) load_pages(t0, ke * kPlanBlock);
     int L, first, pieces, slot;
     sload_request(p.seq_lens + rb, req_info + 3 * (int64_t)rb, L, first, pieces, slot);
-    const int t1 = max(t0, bounded ? min(ke * kPlanBlock, L) : L);
+    const int t1 = max(t0, re == rb ? min(ke * kPlanBlock, L) : L);
     if (tid == 0) {
       s.t0[0] = t0;
       s.t1[0] = t1;
@@ -67,7 +64,7 @@ __device__ __forceinline__ void stage_range(const DecodeParams& p, int rb, int k
       s.slot0[0] = slot - first;
     }
     if constexpr (kPages) {
-      if (!bounded) load_pages(t0, t1);
+      load_pages(t0, t1);
 #pragma unroll
       for (int u = 0; u < kPer; ++u) {
         const int k = tid + kThreads * u;

@@ -117,3 +117,27 @@ def test_decode_head_counts_beyond_32_bit_offsets():
         out, lse = _decode(q, pool, pt, lens, 1, 12)
         torch.testing.assert_close(out.float(), o_ref, **O_TOL)
         torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
+
+
+@pytest.mark.parametrize("heads", [8, 24, 64, 130])
+@pytest.mark.parametrize("ps", [32, 64])
+def test_decode_page_table_row_stride_is_not_its_width(heads, ps):
+    """A one-row table made by a transpose has strides (1, 1), and rows that overlap have a stride below their
+    width: neither bounds the columns. 16 plan ranges: most lie inside one request, its last one among them."""
+    print(f"[decode table stride] heads={heads} ps={ps}", flush=True)
+    case = make_decode_case(1, heads, ps, lens=[1500], seed=heads + ps)
+    pt = case.page_table.view(-1, 1).to(DEV).t()
+    assert pt.stride() == (1, 1) and pt.shape[1] > 1
+    out, lse = _decode(case.q, case.kv_pool, pt, [1500], ps, 16)
+    o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, [1500])
+    torch.testing.assert_close(out.float(), o_ref, **O_TOL)
+    torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
+    lens = [1400, 900, 1300]  # row b is the ids from 2b on
+    ids = torch.cat([case.page_table[0].to(torch.int32), case.page_table[0, :4].to(torch.int32)])
+    pt = ids.to(DEV).as_strided((3, case.page_table.shape[1]), (2, 1))
+    q = case.q.expand(3, heads, 576).clone()
+    q[1:] = -q[1:]
+    out, lse = _decode(q, case.kv_pool, pt, lens, ps, 16)
+    o_ref, lse_ref = R.mla_decode(q, case.kv_pool, pt.cpu(), lens)
+    torch.testing.assert_close(out.float(), o_ref, **O_TOL)
+    torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
