@@ -141,3 +141,21 @@ def test_decode_page_table_row_stride_is_not_its_width(heads, ps):
     o_ref, lse_ref = R.mla_decode(q, case.kv_pool, pt.cpu(), lens)
     torch.testing.assert_close(out.float(), o_ref, **O_TOL)
     torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
+
+
+@pytest.mark.parametrize("heads,num_ctas", [(8, 1), (16, 3), (24, 1), (64, 1)])
+def test_decode_tokens_of_infinitely_low_score(heads, num_ctas):
+    """Tokens that a query scores -inf (a rope dim of -inf) count for nothing, also where they fill a piece's first
+    tile, whose maximum is the exponent reference."""
+    lens = [100, 700]
+    case = make_decode_case(2, heads, 64, lens=lens, seed=heads)
+    kv = case.kv_pool.float()
+    for b, L in enumerate(lens):
+        kv.view(-1, 576)[R.token_rows(case.page_table[b], L, 64)[:70], 512] = -float("inf")
+    case.kv_pool = kv.to(torch.bfloat16)
+    case.q[..., 512] = 1.0
+    out, lse = _decode(case.q, case.kv_pool, case.page_table, lens, 64, num_ctas)
+    o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, lens)
+    assert torch.isfinite(o_ref).all()
+    torch.testing.assert_close(out.float(), o_ref, **O_TOL)
+    torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
