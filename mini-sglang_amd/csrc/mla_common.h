@@ -57,6 +57,14 @@ struct DecodeParams {
   int64_t lse_stride_b;
 };
 
+// The streaming decode kernels hold row offsets in 32 bits: of a tile's queries (tile_heads of them at most) from its
+// first and, with pages under 32 tokens, of every pool row from the pool's base. The general kernel takes any.
+inline bool row_offsets_fit(const DecodeParams& p, int tile_heads) {
+  const int64_t span = (p.heads < tile_heads ? p.heads : tile_heads) - 1;
+  if (span * p.q_stride_h * 2 + kRowBytes > (int64_t)UINT32_MAX) return false;
+  return p.log2_ps >= 5 || ((int64_t)p.num_pages << p.log2_ps) * p.kv_row_stride * 2 <= (int64_t)UINT32_MAX;
+}
+
 struct MergeParams {
   const __bf16* ws_o;  // bf16 partials, chunk order of mla_amd.h
   const float* ws_lse;
@@ -117,11 +125,11 @@ hipError_t launch_prefill_gather(const void* kv, int64_t kv_row_stride, int32_t 
                                  int64_t c_row_stride, void* rope_out, int64_t rope_row_stride, int64_t out_rows,
                                  int32_t* seg_pt, int64_t seg_pt_stride, hipStream_t stream);
 hipError_t launch_decode(const DecodeParams& p, hipStream_t stream);
-// The warp-specialized kernel: 64 heads, any power-of-two page size (under 32 tokens only while every
-// row offset of the pool fits in 32 bits).
+// The warp-specialized kernel: 17 heads and more (past 64 in groups of 64, one launch), any power-of-two page size,
+// while row offsets fit in 32 bits.
 bool decode_ws_takes(const DecodeParams& p);
 hipError_t launch_decode_ws(const DecodeParams& p, hipStream_t stream);
-// The few-heads kernel: up to 32 heads, any power-of-two page size (with the same bound on the pool).
+// The few-heads kernel: up to 16 heads, any power-of-two page size, with the same bound on row offsets.
 bool decode_fh_takes(const DecodeParams& p);
 hipError_t launch_decode_fh(const DecodeParams& p, hipStream_t stream);
 hipError_t launch_merge(const MergeParams& p, hipStream_t stream);

@@ -2,8 +2,8 @@
 // merge of the split partials (bf16 partial outputs, fp32 LSEs).
 //
 // The general kernel runs what neither the few-heads kernel (up to 16 heads) nor the warp-specialized one
-// (17 heads and more) takes: pages of fewer than 32 tokens in a pool past 4 GiB, whose row offsets need 64
-// bits.
+// (17 heads and more) takes: row offsets that need 64 bits, those of pages under 32 tokens in a pool past 4 GiB and
+// of queries whose heads lie so far apart that 16 or 32 of them span 4 GiB.
 //
 // Work decomposition: a CTA (one wave per 16 query heads) owns one contiguous
 // range of (request, 64-token block) space from the host plan. For each piece

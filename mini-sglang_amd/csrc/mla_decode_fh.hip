@@ -390,12 +390,7 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
 
 }  // namespace
 
-bool decode_fh_takes(const DecodeParams& p) {
-  if (p.heads < 1 || p.heads > 16) return false;
-  if (p.log2_ps >= 5) return true;
-  // pages under 32 tokens: every row offset from the pool base must fit in 32 bits
-  return ((int64_t)p.num_pages << p.log2_ps) * p.kv_row_stride * 2 <= (int64_t)UINT32_MAX;
-}
+bool decode_fh_takes(const DecodeParams& p) { return p.heads >= 1 && p.heads <= 16 && row_offsets_fit(p, 16); }
 
 hipError_t launch_decode_fh(const DecodeParams& p, hipStream_t stream) {
   const int cus = current_device_cus();

@@ -631,12 +631,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
 
 }  // namespace
 
-bool decode_ws_takes(const DecodeParams& p) {
-  if (p.heads <= 16) return false;
-  if (p.log2_ps >= 5) return true;
-  // pages under 32 tokens: every row offset from the pool base must fit in 32 bits
-  return ((int64_t)p.num_pages << p.log2_ps) * p.kv_row_stride * 2 <= (int64_t)UINT32_MAX;
-}
+bool decode_ws_takes(const DecodeParams& p) { return p.heads > 16 && row_offsets_fit(p, 32); }
 
 template <bool kSmall>
 static void launch_ws(const DecodeParams& p, hipStream_t stream) {

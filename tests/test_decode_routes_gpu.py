@@ -1,9 +1,9 @@
 """Head counts and page sizes at the edges of the decode dispatch, against the CPU oracle.
 
 Up to 16 heads run the few-heads kernel, 17..63 the warp-specialized kernel padded to 64, more than 64 its
-groups of 64 in one launch (the last group padded), and any count the general kernel when pages are under
-32 tokens and the pool's row offsets do not fit in 32 bits. Tolerances: bf16 output atol = rtol = 2e-2, fp32
-LSE atol 1e-3 (as everywhere in the decode tests).
+groups of 64 in one launch (the last group padded), and any count the general kernel when row offsets do not fit
+in 32 bits (of the queries, or of the pool with pages under 32 tokens). Tolerances: bf16 output atol = rtol = 2e-2,
+fp32 LSE atol 1e-3 (as everywhere in the decode tests).
 """
 
 from __future__ import annotations
@@ -157,5 +157,22 @@ def test_decode_tokens_of_infinitely_low_score(heads, num_ctas):
     out, lse = _decode(case.q, case.kv_pool, case.page_table, lens, 64, num_ctas)
     o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, lens)
     assert torch.isfinite(o_ref).all()
+    torch.testing.assert_close(out.float(), o_ref, **O_TOL)
+    torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
+
+
+
+@pytest.mark.parametrize("heads,ps,stride", [(16, 64, 150_000_000), (20, 64, 120_000_000), (32, 1, 72_000_000),
+                                             (70, 64, 72_000_000)])
+def test_decode_query_rows_beyond_32_bit_offsets(heads, ps, stride):
+    """Heads of a query so far apart that a tile of 16 or 32 of its rows spans more than 4 GiB."""
+    print(f"[decode query stride] heads={heads} ps={ps}", flush=True)
+    lens = [300]
+    case = make_decode_case(1, heads, ps, lens=lens, seed=heads)
+    q = torch.empty((heads - 1) * stride + 576, dtype=torch.bfloat16, device=DEV).as_strided(
+        (1, heads, 576), (heads * stride, stride, 1))
+    q.copy_(case.q)
+    out, lse = _decode(q, case.kv_pool, case.page_table, lens, ps, 3)
+    o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, lens)
     torch.testing.assert_close(out.float(), o_ref, **O_TOL)
     torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
