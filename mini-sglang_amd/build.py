@@ -2,7 +2,8 @@
 
 Usage: python mini-sglang_amd/build.py [--jobs N]
 The library lands in minisgl_amd/kernel/libmla_amd.so, where
-minisgl_amd.kernel.lib loads it. Every call recompiles.
+minisgl_amd.kernel.lib loads it. Every call recompiles, and
+fails if the device assembly breaks a wait-state rule (asm_check.py).
 """
 
 from __future__ import annotations
@@ -15,6 +16,10 @@ import subprocess
 import sys
 
 HERE = os.path.dirname(os.path.abspath(__file__))
+if HERE not in sys.path:
+    sys.path.insert(0, HERE)
+import asm_check  # noqa: E402
+
 CSRC = os.path.join(HERE, "csrc")
 BUILD = os.path.join(HERE, "_build")
 OUT = os.path.join(HERE, "minisgl_amd", "kernel", "libmla_amd.so")
@@ -39,9 +44,19 @@ FLAGS = [
 SOURCE_FLAGS = {"mla_prefill.hip": ["-Xarch_device", "-fno-honor-nans"]}
 
 
+def check_assembly(name: str, asm: str) -> None:
+    """Raises if the device assembly of source ``name`` breaks a rule of ``asm_check``: such code loads from wrong
+    addresses and can fault the GPU."""
+    sgpr, m0 = asm_check.find_hazards(asm)
+    found = sgpr + m0 + asm_check.find_lane_read_hazards(asm)
+    if found:
+        raise RuntimeError(f"{name}: {len(found)} missing wait states in the device assembly: {found[:3]}")
+
+
 def _compile(src: str) -> str:
-    obj = os.path.join(BUILD, os.path.basename(src) + ".o")
-    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(os.path.basename(src), []), "-c", src, "-o", obj]
+    name = os.path.basename(src)
+    obj = os.path.join(BUILD, name + ".o")
+    cmd = [HIPCC, *FLAGS, *SOURCE_FLAGS.get(name, []), "--save-temps=obj", "-c", src, "-o", obj]
     res = subprocess.run(cmd, capture_output=True, text=True)
     noise = "'-packed-fp32-ops' is not a recognized feature"
     err = "\n".join(l for l in res.stderr.splitlines() if noise not in l)
@@ -49,6 +64,8 @@ def _compile(src: str) -> str:
         raise RuntimeError(f"hipcc failed for {src}:\n{err}")
     if err.strip():
         print(err, file=sys.stderr)
+    with open(os.path.join(BUILD, f"{name.removesuffix('.hip')}-hip-amdgcn-amd-amdhsa-{ARCH}.s")) as f:
+        check_assembly(name, f.read())
     return obj
 
 

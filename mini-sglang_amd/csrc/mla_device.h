@@ -79,31 +79,35 @@ __device__ __forceinline__ void wait_vmcnt() {
 // pass does not serialise later LDS reads of other stages behind it: every
 // read of a staged tile is preceded by wait_vmcnt + a workgroup barrier.
 // The compiler's hazard recognizer does not look inside inline asm, so the
-// wait states it would add are written here: an LDS DMA reads M0 one wait
-// state after a scalar write of M0 (the compiler writes M0 just before the
-// asm statement).
+// wait states it would add are written here: one between a scalar write of
+// M0 (the compiler writes it just before the statement) and an LDS DMA. The
+// base's scalar registers need five after a vector-ALU write: uniform_ptr
+// waits them out, and the build checks the assembly for any other write (a
+// spilled base's v_readlane), which this statement could not survive (waits of
+// its own here cost a prefill step 1.3 %).
 __device__ __forceinline__ void dma16_saddr(const char* base, uint32_t voff, uint32_t lds_base) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(base), "{m0}"(lds_base) : "memory");
 }
-// Load of column block B (128 B bytes into the row, B KiB x 4 into the tile): the immediate offset is added to the
-// source and to the LDS address, so the LDS base gives it back. kNt: the non-temporal hint, for data read once
-// (streamed KV rows), so the caches keep the lines that are reused.
-template <int B, bool kNt>
-__device__ __forceinline__ void dma16_block(const char* base, uint32_t voff, uint32_t lds_base) {
-  const uint32_t m0 = lds_base + B * (kTileBlockBytes - 128);
-  if constexpr (kNt)
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3 nt" ::"v"(voff), "s"(base), "{m0}"(m0), "n"(B * 128) : "memory");
-  else
-    asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%3" ::"v"(voff), "s"(base), "{m0}"(m0), "n"(B * 128) : "memory");
-}
-// All blocks of a token octet: one wave's 9 loads of a tile.
-template <bool kNt, int B = 0>
+// All column blocks of a token octet, one wave's 9 loads of a tile, as one statement that waits for its own base: a
+// base restored from a spill by a v_readlane right before the loads is then safe (with one statement per load, such a
+// restore loaded from a wild address). Block B lies 128 B bytes into the row and 4096 B bytes into the tile; the immediate offset is
+// added to the source and to the LDS address, so M0 steps by the difference. kNt: the non-temporal hint, for data
+// read once (streamed KV rows), so the caches keep the lines that are reused.
+#define MLA_DMA_BLOCK(offset, hint) \
+  "s_add_u32 m0, m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:" #offset hint "\n\t"
+#define MLA_DMA_OCTET(hint)                                                                                       \
+  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %1, %2" hint "\n\t" MLA_DMA_BLOCK(128, hint)               \
+               MLA_DMA_BLOCK(256, hint) MLA_DMA_BLOCK(384, hint) MLA_DMA_BLOCK(512, hint) MLA_DMA_BLOCK(640, hint) \
+               MLA_DMA_BLOCK(768, hint) MLA_DMA_BLOCK(896, hint) MLA_DMA_BLOCK(1024, hint)                         \
+               : "+{m0}"(lds_base) : "v"(voff), "s"(base), "n"(kTileBlockBytes - 128) : "scc", "memory")
+template <bool kNt>
 __device__ __forceinline__ void dma16_octet(const char* base, uint32_t voff, uint32_t lds_base) {
-  if constexpr (B < kTileBlocks) {
-    dma16_block<B, kNt>(base, voff, lds_base);
-    dma16_octet<kNt, B + 1>(base, voff, lds_base);
-  }
+  static_assert(kTileBlocks == 9, "one load per column block");
+  if constexpr (kNt) MLA_DMA_OCTET(" nt");
+  else MLA_DMA_OCTET("");
 }
+#undef MLA_DMA_OCTET
+#undef MLA_DMA_BLOCK
 __device__ __forceinline__ void dma16_vaddr(const char* addr, uint32_t lds_base) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(addr), "{m0}"(lds_base) : "memory");
 }

@@ -10,53 +10,13 @@ kernel source, over every control-flow path (no GPU needed).
 from __future__ import annotations
 
 import os
-import re
 import sys
-from typing import Set
 
 import pytest
 
 sys.path.insert(0, os.path.dirname(os.path.abspath(__file__)))
 import test_asm_hazards_cpu as asm_check  # noqa: E402
-
-
-def _vgprs(text: str) -> Set[int]:
-    regs = set()
-    for m in re.finditer(r"\bv\[(\d+):(\d+)\]", text):
-        regs.update(range(int(m.group(1)), int(m.group(2)) + 1))
-    regs.update(int(m.group(1)) for m in re.finditer(r"\bv(\d+)\b", text))
-    return regs
-
-
-def _valu_dests(line: str) -> Set[int]:
-    op = line.split()[0]
-    if not op.startswith("v_") or op.startswith(("v_cmp", "v_readfirstlane", "v_readlane")):
-        return set()
-    ops = asm_check._operands(line)
-    both = op.startswith("v_swap") or ("permlane" in op and "swap" in op)
-    return _vgprs(" ".join(ops[: 2 if both else 1]))
-
-
-def find_lane_read_hazards(asm: str):
-    found = []
-    for fn in asm_check.functions(asm):
-        for b, ins in enumerate(fn.blocks):
-            for i, line in enumerate(ins):
-                if not line.startswith(("v_readfirstlane_b32", "v_readlane_b32")):
-                    continue
-                reads = _vgprs(asm_check._operands(line)[1])
-                before, stack, seen = [], [(b, i)], set()
-                while stack:  # the instruction before, on every path
-                    blk, at = stack.pop()
-                    if at > 0:
-                        before.append(fn.blocks[blk][at - 1])
-                        continue
-                    for p in fn.preds[blk]:
-                        if p not in seen:
-                            seen.add(p)
-                            stack.append((p, len(fn.blocks[p])))
-                found += [(fn.name, w, line) for w in before if _valu_dests(w) & reads]
-    return list(dict.fromkeys(found))
+from asm_check import find_lane_read_hazards  # noqa: E402
 
 
 def test_checker_catches_a_lane_read_right_after_the_write():
