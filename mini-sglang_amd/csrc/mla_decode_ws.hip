@@ -65,19 +65,23 @@ struct WCursor {
 // step's barrier, when they issue the tile. The launcher takes this path only when every row offset
 // of the pool fits in 32 bits.
 //
-// kLoop: the launch has fewer CTAs than the plan has ranges (a plan laid out for a larger grid, as a
-// captured decode step's is); CTA b then runs ranges b, b + gridDim.x, ... in turn and stops at the
-// first padding range. Without it (at most one range per compute unit) each CTA runs range blockIdx.x
-// and the body has no loop around it: the loop makes the compiler keep values across both roles'
-// step loops and spill.
+// kLoop: the plan has more than two ranges per compute unit (one laid out for a larger grid, as a captured decode
+// step's is); the launch has one CTA per compute unit (and group), which runs its range and every n-th after it in
+// turn and stops at the first padding range. Without it each CTA runs one range and the body has no loop around it
+// (the loop makes the compiler keep values across both roles' step loops and spill). A padding range then costs a
+// CTA that takes a compute unit's LDS to find it has nothing to do. Split step, loop-free / loop: 128 heads, 32
+// requests of 1k to 8k tokens in 256 ranges of a plan for 512: 65.7 / 66.5 us, for 2048: 70.7-74.6 / 66.5; 32
+// heads, 64 requests, for 2048: 66.0 / 64.0; one request of 1,500 tokens, 64 heads, for 512: 9.4 / 10.0; 40 requests
+// of 960 to 1,120 tokens in 341 ranges, 24 heads 23.9 / 24.6, 64 heads 26.7 / 27.0, 128 heads 40.1 / 41.3.
 // kMode kPadded: 17 to 63 heads; query rows past the last head load the last head again and their outputs are
 // not written (the padding costs MFMAs, which the KV stream hides: 32 heads, 64 requests of 1k to 8k tokens,
 // 67.9 us against 78.1 us on the general kernel; 48 heads 70.7 against 82.5 us).
-// kMode kGroups: more than 64 heads, in groups of 64 (the last one padded): CTA blockIdx.x runs one group of one range, and the groups of a range are CTAs 8 apart, which the dispatcher
-// puts on the same XCD at about the same time: the range's KV tiles come from HBM once and from that XCD's
-// L2 for the other groups (so they are loaded without the non-temporal hint). One launch per group, each
-// streaming the KV from HBM, took 80.8 us for 128 heads, 32 requests of 1k to 8k tokens, where this took 77.2 us
-// (and 66 us with the tile layout and waits of today; HBM no longer bounds it).
+// kMode kGroups: more than 64 heads, in groups of 64 (the last one padded): a CTA runs one group of one range, and
+// the groups of a range are CTAs 8 apart, which the dispatcher puts on the same XCD at about the same time: the
+// range's KV tiles come from HBM once and from that XCD's L2 for the other groups (so they are loaded without the
+// non-temporal hint). One launch per group, each streaming the KV from HBM, took 80.8 us for 128 heads, 32 requests
+// of 1k to 8k tokens, where this took 77.2 us (and 66 us with the tile layout and waits of today; HBM no longer
+// bounds it).
 enum WMode { kExact, kPadded, kGroups };
 
 template <bool kSmall, bool kLoop, WMode kMode>
@@ -617,8 +621,9 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
   };
 
   if constexpr (kLoop) {
-    for (int w = blockIdx.x; w < p.num_ctas; w += gridDim.x) {
-      if (w != (int)blockIdx.x) {  // the previous range's waves are done with the LDS tables and ring
+    const int step = kMode == kGroups ? (int)gridDim.x / ((p0.heads + 63) >> 6) : (int)gridDim.x;
+    for (int w = w_first; w < p.num_ctas; w += step) {
+      if (w != w_first) {  // the previous range's waves are done with the LDS tables and ring
         wait_vmcnt<0>();
         __syncthreads();
       }
@@ -633,20 +638,22 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
 
 bool decode_ws_takes(const DecodeParams& p) { return p.heads > 16 && row_offsets_fit(p, 32); }
 
+template <bool kSmall, WMode kMode>
+static void launch_mode(const DecodeParams& p, int groups, hipStream_t stream) {
+  const int cus = current_device_cus();
+  const bool loop = p.num_ctas > 2 * cus;  // measured at kLoop
+  int ctas = loop ? cus : p.num_ctas;
+  if (kMode == kGroups) ctas = (ctas + 7) / 8 * 8;  // ranges in eights (one per XCD)
+  const dim3 grid(ctas * groups), threads(kWWaves * 64);
+  if (loop) hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, true, kMode>), grid, threads, 0, stream, p);
+  else hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, false, kMode>), grid, threads, 0, stream, p);
+}
+
 template <bool kSmall>
 static void launch_ws(const DecodeParams& p, hipStream_t stream) {
-  const int cus = current_device_cus();
-  const dim3 threads(kWWaves * 64);
-  if (p.heads > 64) {  // one CTA per (range, 64-head group); ranges in eights (one per XCD)
-    const int grid = (p.num_ctas + 7) / 8 * 8 * ((p.heads + 63) / 64);
-    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, false, kGroups>), dim3(grid), threads, 0, stream, p);
-  } else if (p.heads < 64) {
-    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, false, kPadded>), dim3(p.num_ctas), threads, 0, stream, p);
-  } else if (p.num_ctas <= cus) {
-    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, false, kExact>), dim3(p.num_ctas), threads, 0, stream, p);
-  } else {
-    hipLaunchKernelGGL((mla_decode_ws_kernel<kSmall, true, kExact>), dim3(cus), threads, 0, stream, p);
-  }
+  if (p.heads > 64) launch_mode<kSmall, kGroups>(p, (p.heads + 63) / 64, stream);
+  else if (p.heads < 64) launch_mode<kSmall, kPadded>(p, 1, stream);
+  else launch_mode<kSmall, kExact>(p, 1, stream);
 }
 
 hipError_t launch_decode_ws(const DecodeParams& p, hipStream_t stream) {

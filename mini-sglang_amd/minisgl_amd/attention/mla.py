@@ -366,9 +366,9 @@ class MLAAttnBackend(BaseAttnBackend):
         # the captured launch has a fixed plan grid: the one the largest batch the graphs can replay
         # needs. Its tokens are bounded by max_bs * max_seq_len, not by the pool: requests sharing
         # prefix pages (the radix cache) can hold more tokens in all than the pool has. The kernels
-        # run a plan of more ranges than compute units as a loop over ranges (the launch grid stays
-        # at one CTA per compute unit) and stop at the first padding range, so a large plan grid costs
-        # only its workspace (2 slots per range)
+        # run a plan of more than two ranges per compute unit as a loop over ranges (one CTA per compute
+        # unit) and stop at the first padding range, so a large plan grid costs its workspace (2 slots
+        # per range) and up to 1 us of a short step
         self.capture_ctas = plan_grid_bound(self.num_ctas, max_bs * max_seq_len, max_bs)
         plan = torch.zeros((self.capture_ctas * lib.PLAN_CTA_INTS + max_bs * lib.PLAN_REQ_INTS,), dtype=torch.int32,
                            device=self.device)

@@ -176,3 +176,20 @@ def test_decode_query_rows_beyond_32_bit_offsets(heads, ps, stride):
     o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, lens)
     torch.testing.assert_close(out.float(), o_ref, **O_TOL)
     torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
+
+
+@pytest.mark.parametrize("heads,ps", [(8, 64), (8, 1), (24, 32), (40, 1), (64, 64), (100, 64), (130, 8)])
+def test_decode_second_range_of_a_cta(heads, ps):
+    """A plan of more non-empty ranges than compute units, padded to 600: a CTA runs one range after another through
+    the same LDS ring and tables (the row-offset ring with small pages), and stops at the first padding range."""
+    print(f"[decode loop] heads={heads} ps={ps}", flush=True)
+    lens = [960 + (37 * i) % 160 for i in range(40)]
+    cus = lib.device_cu_count(torch.cuda.current_device())
+    plan, _ = lib.decode_plan(lens, ps, 600)
+    used = int((plan[: 4 * 600].reshape(600, 4)[:, 0] < len(lens)).sum())
+    assert cus < used < 600 and 600 > 2 * cus
+    case = make_decode_case(len(lens), heads, ps, lens=lens, seed=heads + ps)
+    out, lse = _decode(case.q, case.kv_pool, case.page_table, lens, ps, 600)
+    o_ref, lse_ref = R.mla_decode(case.q, case.kv_pool, case.page_table, lens)
+    torch.testing.assert_close(out.float(), o_ref, **O_TOL)
+    torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
