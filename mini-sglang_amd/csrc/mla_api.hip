@@ -335,6 +335,7 @@ static mla::MergeParams merge_params(const __bf16* ws_o, const float* ws_lse, in
   m.batch = batch;
   m.heads = heads;
   m.skip_single = skip_single;
+  m.likely_slots = ws_slots;
   m.out = static_cast<__bf16*>(out);
   m.out_stride_b = out_stride_b;
   m.out_stride_h = out_stride_h;
@@ -470,8 +471,12 @@ int decode_split_merge(const char* who, const void* q, int64_t q_stride_b, int64
                                pt_stride, seq_lens, batch, heads, scale, plan, num_ctas, ws_o, ws_lse, ws_slots, out,
                                out_stride_b, out_stride_h, lse, lse_stride_b, stream))
     return rc;
-  const MergeParams m = merge_params(ws_o, ws_lse, ws_slots, plan + 4 * (int64_t)num_ctas, batch, heads, 1, out,
-                                     out_stride_b, out_stride_h, lse, lse_stride_b);
+  MergeParams m = merge_params(ws_o, ws_lse, ws_slots, plan + 4 * (int64_t)num_ctas, batch, heads, 1, out,
+                               out_stride_b, out_stride_h, lse, lse_stride_b);
+  // The plan is on the device. A range boundary or a request's end closes a piece, so a plan has at most a slot per
+  // range and request, however large the workspace; ranges past one per compute unit are mostly padding.
+  const int64_t ranges = std::min(num_ctas, current_device_cus());
+  m.likely_slots = (int32_t)std::min<int64_t>(ws_slots, ranges + batch);
   return hip_status(mla::launch_merge(m, (hipStream_t)stream), "decode merge launch");
 }
 

@@ -72,6 +72,7 @@ struct MergeParams {
   const int32_t* req_info;  // [batch * 3]
   int32_t batch, heads;
   int32_t skip_single;  // requests with one piece were finalised by the decode kernel
+  int32_t likely_slots;  // slots that the plan's requests are taken to have in all (chooses the launch, no more)
   __bf16* out;
   int64_t out_stride_b, out_stride_h;
   float* lse;

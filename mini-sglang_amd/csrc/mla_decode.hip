@@ -321,11 +321,14 @@ __global__ __launch_bounds__(NW * 64, 1) void mla_decode_kernel(const DecodePara
 // arithmetic, one rounding to bf16; piece i is added to partial sum i % 4 for either kWaves, so both give the
 // same bits.
 // Bound: latency (launch, plan entry, partials, output), so four waves pay where a request has more pieces
-// than one wave reads in a round trip. Step time less the split step's, 64 heads: one request in 23 pieces
-// 8.3 -> 3.8 us, 8 of 1k to 8k tokens 11.3 -> 5.4 us, 8 of 32k to 128k tokens 9.9 -> 3.9 us; at 8 slots per
-// request (32 requests, 128 heads) one wave is the faster by 1.4 us, at 10.7 (24 requests) four by 1.3 us.
+// than one wave reads in a round trip, and fewer heads leave room for more waves. Step less split step, 64 heads,
+// one wave -> four: one request in 23 pieces 8.3 -> 3.8 us, 8 of 1k to 8k tokens 11.3 -> 5.4 us, 8 of 32k to 128k
+// tokens 9.9 -> 3.9 us. Whole step by likely slots per request, one wave / four: 64 heads 13.8: 34.9 / 33.0 us,
+// 10.1: 41.4 / 40.8, 9.0: 44.9 / 44.9, 8.1: 47.6 / 48.1, 6.8: 53.5 / 55.1; 128 heads 10.8: 67.5 / 67.3,
+// 9.0: 78.3 / 79.4, 6.8: 94.9 / 97.9; 16 heads 9.0: 38.8 / 37.6, 8.1: 41.4 / 40.4, 6.8: 47.9 / 47.7.
 constexpr int kMergeBatch = 8;
-constexpr int kMergeWideSlots = 10;  // workspace slots per request from which four waves merge a head
+constexpr int kMergeWideSlots = 10, kMergeWideSlotsFew = 7;  // slots per request from which four waves merge a head,
+constexpr int kMergeFewHeads = 16;                           // above and up to this many heads
 
 __device__ __forceinline__ void unpack_bf16x8(const u32x4 raw, float* f) {
 #pragma unroll
@@ -457,8 +460,8 @@ hipError_t launch_decode(const DecodeParams& p, hipStream_t stream) {
 }
 
 hipError_t launch_merge(const MergeParams& p, hipStream_t stream) {
-  // The plan is on the device; the workspace's slots bound the pieces of an average request.
-  if ((int64_t)p.ws_slots >= (int64_t)kMergeWideSlots * p.batch && p.heads <= 65535)
+  const int64_t wide = p.heads <= kMergeFewHeads ? kMergeWideSlotsFew : kMergeWideSlots;
+  if (p.likely_slots >= wide * p.batch && p.heads <= 65535)
     hipLaunchKernelGGL(mla_merge_kernel<4>, dim3(p.batch, p.heads), dim3(256), 0, stream, p);
   else
     hipLaunchKernelGGL(mla_merge_kernel<1>, dim3(p.batch, (p.heads + 3) / 4), dim3(256), 0, stream, p);
