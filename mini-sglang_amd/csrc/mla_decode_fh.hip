@@ -36,7 +36,7 @@ constexpr int kFKPrefetch = 6;  // K operands in flight
 constexpr int kFVPrefetch = 4;  // V operand pairs in flight
 constexpr int kFMaxTiles = 2 * kMaxCtaBlocks;
 constexpr float kFRescaleLog2 = 64.0f;
-// The lowest exponent reference: a first tile whose scores are all -inf then has numerators of zero, and the first
+// The lowest maximum of a tile: where all scores of a first tile are -inf its numerators are then zero, and the first
 // finite score moves the reference (against -inf the numerators, and with them the whole piece, would be NaN).
 constexpr float kFLowest = -3.402823466e38f;
 static_assert(kFAhead == kStages - 1 && kFAhead == 3, "a tile is issued into the stage of the tile just finished");
@@ -278,7 +278,7 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
           vhi[db] = vread(db, 1);
         }
         const int valid = cs.t1 - cs.t;
-        float x[8], mt = -INFINITY;
+        float x[8], mt = kFLowest;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
           x[i] = sv[i >> 2][i & 3] * p.scale_log2;
@@ -286,7 +286,7 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
           mt = fmaxf(mt, x[i]);
         }
         if (cs.t == cs.t0) {
-          m_ref = fmaxf(wave_max_g(mt), kFLowest);
+          m_ref = wave_max_g(mt);
         } else if (__ballot(mt > m_ref + kFRescaleLog2) != 0) {  // rare, and the same in every wave
           const float m_new = fmaxf(wave_max_g(mt), m_ref);
           const float f = __builtin_amdgcn_exp2f(m_ref - m_new);
@@ -325,7 +325,7 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
           const bool to_ws = npieces != 1;
           const float l = wave_sum_g(l_run);
           // no score above -inf: nothing to the merge, and no result (NaN) for a whole request
-          const float inv = l > 0.f ? 1.f / l : (to_ws ? 0.f : __builtin_nanf(""));
+          const float inv = to_ws && !(l > 0.f) ? 0.f : 1.f / l;
           const float lse_nat = l > 0.f ? (m_ref + log2f(l)) * 0.69314718055994531f : -INFINITY;
           if (to_ws) {
             if (slot >= 0 && slot < p.ws_slots) {
