@@ -4,6 +4,8 @@ of the rule that chooses between them, against the CPU oracle; tolerances as in 
 
 from __future__ import annotations
 
+import copy
+
 import pytest
 import torch
 
@@ -38,13 +40,30 @@ def _check(case):
 @pytest.mark.parametrize("heads,ps,extends,prefixes", [
     (3, 64, [1], [0]), (2, 64, [128], [0]), (2, 64, [129], [31]), (5, 128, [127, 1, 130], [1, 1000, 33]),
     (1, 64, [20], [100]),  # a last stage of 24 keys, and waves without rows
-    (1, 64, [70], [16500]),  # more stages than the 128-row CTA stages sources for
+    (1, 64, [70], [16500]), (2, 128, [130], [33000]),  # a second and a third window of stage sources
     (70, 64, [700, 641], [65, 0]),  # 256-row CTAs: over 640 rows a request and more than 256 of them
     (90, 64, [641], [32 * 9 + 5]),  # the first size past the rule's line
 ])
 def test_prefill_cta_shapes(heads, ps, extends, prefixes):
     print(f"[prefill shapes] heads={heads} ps={ps} {extends} {prefixes}", flush=True)
     _check(make_prefill_case(heads, ps, extends=extends, prefixes=prefixes, seed=sum(extends)))
+
+
+def test_prefill_source_windows_of_256_rows():
+    """256-row CTAs over more keys than one window of stage sources (1024 stages, 32,768 keys) holds: bit for bit the
+    128-row CTAs that a launch of one head takes, and some heads against the oracle."""
+    H, E, P = 100, 700, 33500
+    case = make_prefill_case(H, 64, extends=[E], prefixes=[P], device=DEV, seed=21)
+    out, lse = _run(case)
+    for h in (0, 63, 99):
+        head = copy.copy(case)
+        head.q, head.k_pool, head.v_pool = (t[..., h:h + 1, :] for t in (case.q, case.k_pool, case.v_pool))
+        o1, l1 = _run(head)
+        assert torch.equal(o1, out[:, h:h + 1]) and torch.equal(l1, lse[:, h:h + 1])
+        o_ref, lse_ref = R.mla_prefill(head.q.cpu(), head.k_pool.cpu(), head.v_pool.cpu(), case.page_table.cpu(),
+                                       case.cu_seqlens_q.cpu(), case.seq_lens_k.cpu())
+        torch.testing.assert_close(o1, o_ref, **O_TOL)
+        torch.testing.assert_close(l1, lse_ref, **LSE_TOL)
 
 
 def test_prefill_many_requests_of_mixed_lengths():
