@@ -743,13 +743,25 @@ static void launch_shape(const PrefillParams& p, int32_t total_q, hipStream_t st
 // unless said), 256 rows / 128 rows: two requests of 600 rows on 600 keys 73.8 / 65.1 us; 16 of 384 on 1000
 // 402 / 380; six of 1 to 294 rows 55.7 / 52.3; 4 of 700 on 1000 188 / 191; one of 1500 60.7 / 65.5; four of 2048
 // on 4969 to 7961 keys 2278 / 2412; two of 1024 on 1000, 16 heads (128 CTAs of 256 rows) 56.9 / 46.1.
+// Requests of whole 256-row blocks (an average that is a multiple of 256: a scheduler's chunks) have no half-empty
+// ones: from kPrefillLongKeys keys on they take CTAs of 256 rows where these keep more than half of the compute units
+// busy (fewer run faster as twice as many CTAs). The keys are on the device too; the page table's row stride stands for
+// them (it chooses the launch, no more). 256 / 128 rows, 64 heads: eight of 512 rows on 1000 keys 240 / 238 us, on 2000
+// 380 / 385; four of 512 on 8000 612 / 645, on 30,000 2172 / 2297; four of 256 on 8000 (256 CTAs of 256 rows) 337 / 356;
+// one of 512 on 8000 (128) 232 / 187. With other requests 128 rows stay the better choice at any prefix: 700
+// batches of up to 640 rows a request on 3000 to 16,000 keys took 8 % less in the geometric mean than in CTAs of 256,
+// and the worst class, requests of up to 256 rows whose 256-row CTAs just fill the chip, up to 1.33 times as long.
 constexpr int kPrefillSmallRows = 640;
+constexpr int kPrefillLongKeys = 2048;
 
 hipError_t launch_prefill(const PrefillParams& p, int32_t total_q, hipStream_t stream) {
   if (total_q <= 0 || p.heads <= 0 || p.batch <= 0) return hipSuccess;
   const int64_t rows = ((int64_t)total_q + p.batch - 1) / p.batch;  // of an average request
-  const int64_t ctas = (rows + 255) / 256 * p.batch * p.heads;
-  if (rows <= kPrefillSmallRows || ctas <= current_device_cus()) launch_shape<4>(p, total_q, stream);
+  const int64_t ctas = (rows + 255) / 256 * p.batch * p.heads, cus = current_device_cus();
+  const bool whole = (int64_t)total_q % (256 * (int64_t)p.batch) == 0;
+  const bool small = whole && p.pt_stride > (kPrefillLongKeys - 1) >> p.log2_ps ? 2 * ctas <= cus
+                                                                                : rows <= kPrefillSmallRows || ctas <= cus;
+  if (small) launch_shape<4>(p, total_q, stream);
   else launch_shape<8>(p, total_q, stream);
   return hipGetLastError();
 }
