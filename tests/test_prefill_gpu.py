@@ -49,7 +49,7 @@ def test_prefill_ragged(ps):
 
 @pytest.mark.parametrize("heads", [1, 3, 5, 16, 64])
 def test_prefill_heads(heads):
-    """Head counts 1..64, odd ones included (one head per CTA at these sizes)."""
+    """Head counts 1..64, odd ones included."""
     case = make_prefill_case(heads, 64, extends=[129, 64], prefixes=[200, 0], seed=heads)
     check_case(case)
 
@@ -225,12 +225,10 @@ def test_prefill_full_bench_batch_sampled_rows_and_chunking():
 
 
 def test_prefill_head_pairs_odd_heads_chunk_invariant():
-    """A batch large enough for two heads per CTA (one 8192-row extend: 33 row blocks x 63 heads
-    is at least 8 CTAs per compute unit) with an odd head count, so the last CTA of each block
-    runs one head: bit for bit the same as the same rows prefilled as 1024-row chunks, which are
-    small enough to run one head per CTA."""
+    """One 8192-row extend of an odd head count (32 row blocks x 63 heads, 8 CTAs per compute unit): bit for bit the
+    same as the same rows prefilled as 1024-row chunks, which run about one CTA per compute unit."""
     H, E, P, ps = 63, 8192, 300, 64
-    print(f"[prefill head pairs] H={H} E={E} P={P}", flush=True)
+    print(f"[prefill odd heads] H={H} E={E} P={P}", flush=True)
     case = make_prefill_case(H, ps, extends=[E], prefixes=[P], device=DEV, seed=5)
 
     def run(q, cu, lens):
@@ -252,11 +250,10 @@ def test_prefill_head_pairs_odd_heads_chunk_invariant():
 
 
 def test_prefill_head_pairs_unstaged_long_prefix_chunk_invariant():
-    """Two heads per CTA over more stages than the kernel stages sources for (a 30,000-token
-    prefix: the later query blocks read their page ids per stage, so the second head's sources
-    are computed, not moved): bit for bit the same as 1024-row chunks (one head per CTA)."""
+    """More stages than one window of the kernel's stage sources holds (a 30,000-token prefix: the later query blocks
+    fill a second one): bit for bit the same as 1024-row chunks, whose CTAs fill it at other query rows."""
     H, E, P, ps = 64, 8192, 30000, 64
-    print(f"[prefill head pairs, long prefix] H={H} E={E} P={P}", flush=True)
+    print(f"[prefill long prefix] H={H} E={E} P={P}", flush=True)
     case = make_prefill_case(H, ps, extends=[E], prefixes=[P], device=DEV, seed=6)
 
     def run(q, cu, lens):

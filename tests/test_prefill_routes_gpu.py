@@ -37,16 +37,42 @@ def _check(case):
     torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
 
 
+def _cta_rows(case):
+    """Query rows of a CTA by the launcher's rule."""
+    (total, heads, _), batch = case.q.shape, len(case.extends)
+    cus = lib.device_cu_count(torch.cuda.current_device())
+    rows = -(-total // batch)
+    ctas = -(-rows // 256) * batch * heads
+    if total % (256 * batch) == 0 and case.page_table.stride(0) * case.page_size >= 2048:
+        return 128 if 2 * ctas <= cus else 256
+    return 128 if rows <= 640 or ctas <= cus else 256
+
+
 @pytest.mark.parametrize("heads,ps,extends,prefixes", [
     (3, 64, [1], [0]), (2, 64, [128], [0]), (2, 64, [129], [31]), (5, 128, [127, 1, 130], [1, 1000, 33]),
     (1, 64, [20], [100]),  # a last stage of 24 keys, and waves without rows
-    (1, 64, [70], [16500]), (2, 128, [130], [33000]),  # a second and a third window of stage sources
+    (1, 64, [70], [16500]),  # a second window of stage sources
     (70, 64, [700, 641], [65, 0]),  # 256-row CTAs: over 640 rows a request and more than 256 of them
     (90, 64, [641], [32 * 9 + 5]),  # the first size past the rule's line
+    (2, 128, [130], [33000]),  # a third window
 ])
 def test_prefill_cta_shapes(heads, ps, extends, prefixes):
     print(f"[prefill shapes] heads={heads} ps={ps} {extends} {prefixes}", flush=True)
-    _check(make_prefill_case(heads, ps, extends=extends, prefixes=prefixes, seed=sum(extends)))
+    case = make_prefill_case(heads, ps, extends=extends, prefixes=prefixes, seed=sum(extends))
+    assert _cta_rows(case) == (256 if heads >= 70 else 128)
+    _check(case)
+
+
+@pytest.mark.parametrize("cta_rows,heads,extends,prefixes", [
+    (128, 90, [640], [293]),  # the last size up to the line in rows
+    # whole 256-row blocks: more than half of the compute units busy, half of them, and too few keys
+    (256, 70, [256, 256], [1792, 1000]), (128, 64, [256, 256], [1792, 1000]), (128, 70, [256, 256], [1700, 0]),
+])
+def test_prefill_cta_rule(cta_rows, heads, extends, prefixes):
+    print(f"[prefill rule] heads={heads} {extends} {prefixes}", flush=True)
+    case = make_prefill_case(heads, 64, extends=extends, prefixes=prefixes, seed=sum(prefixes))
+    assert _cta_rows(case) == cta_rows
+    _check(case)
 
 
 def test_prefill_source_windows_of_256_rows():
@@ -54,10 +80,12 @@ def test_prefill_source_windows_of_256_rows():
     128-row CTAs that a launch of one head takes, and some heads against the oracle."""
     H, E, P = 100, 700, 33500
     case = make_prefill_case(H, 64, extends=[E], prefixes=[P], device=DEV, seed=21)
+    assert _cta_rows(case) == 256
     out, lse = _run(case)
     for h in (0, 63, 99):
         head = copy.copy(case)
         head.q, head.k_pool, head.v_pool = (t[..., h:h + 1, :] for t in (case.q, case.k_pool, case.v_pool))
+        assert _cta_rows(head) == 128
         o1, l1 = _run(head)
         assert torch.equal(o1, out[:, h:h + 1]) and torch.equal(l1, lse[:, h:h + 1])
         o_ref, lse_ref = R.mla_prefill(head.q.cpu(), head.k_pool.cpu(), head.v_pool.cpu(), case.page_table.cpu(),
@@ -75,10 +103,11 @@ def test_prefill_many_requests_of_mixed_lengths():
         _check(make_prefill_case(2, 64, extends=ext, prefixes=pre, seed=n))
 
 
-@pytest.mark.parametrize("heads,extends", [(4, [40, 200]), (260, [300])])
+@pytest.mark.parametrize("heads,extends", [(4, [40, 200]), (260, [300]), (90, [641])])
 def test_prefill_after_lds_held_nan(heads, extends):
     """The kernel's first value pass has no stage before it and must not count what the LDS held: a decode over NaN
-    rows leaves NaN in every compute unit's LDS, then a prefill over finite inputs runs."""
+    rows leaves NaN in every compute unit's LDS, then a prefill over finite inputs runs (90 heads: in 256-row CTAs,
+    whose V ring has another last slot)."""
     nan = make_decode_case(8, 64, 64, lens=[4096] * 8, seed=1, device=DEV)
     nan.kv_pool.fill_(float("nan"))
     plan_np, slots = lib.decode_plan(nan.lens, 64, 256)
@@ -86,4 +115,6 @@ def test_prefill_after_lds_held_nan(heads, extends):
     out = torch.empty((8, 64, 512), dtype=torch.bfloat16, device=DEV)
     lib.mla_decode(nan.q, nan.kv_pool, nan.page_table, nan.seq_lens, torch.from_numpy(plan_np).to(DEV), 256, ws_o, ws_lse,
                    R.DEFAULT_SCALE, out)
-    _check(make_prefill_case(heads, 64, extends=extends, prefixes=[0] * len(extends), seed=9))
+    case = make_prefill_case(heads, 64, extends=extends, prefixes=[0] * len(extends), seed=9)
+    assert _cta_rows(case) == (256 if heads == 90 else 128)
+    _check(case)
