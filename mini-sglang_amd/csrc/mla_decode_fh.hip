@@ -67,7 +67,7 @@ __global__ __launch_bounds__((kFWaves + (kSmall ? 1 : 0)) * 64, 1) void mla_deco
   const int H = p.heads;
   const int ps_mask = (1 << p.log2_ps) - 1;
   const int row_bytes = (int)(p.kv_row_stride * 2);
-  const int qrow_bytes = (int)(p.q_stride_h * 2);
+  const uint32_t qrow_bytes = (uint32_t)(p.q_stride_h * 2);
   const char* kv = reinterpret_cast<const char*>(p.kv);
   const uint32_t lds_ring = (uint32_t)(uintptr_t)(MLA_LDS char*)smem;
 

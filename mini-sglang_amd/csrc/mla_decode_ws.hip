@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kWWaves * 64, 1) void mla_decode_ws_kernel(const De
     // that they land while the range is staged (the staging's barriers wait on LDS only). If the
     // first piece turns out to be another request's, the stream issues its query tiles into the same
     // stages after these loads, and loads of one wave complete in order.
-    const int qrow_bytes = (int)(p.q_stride_h * 2);
+    const uint32_t qrow_bytes = (uint32_t)(p.q_stride_h * 2);
     auto issue_query = [&](int b, int qt, uint32_t stage) {  // this output wave's octet of query tile qt of request b
       const char* qsrc = reinterpret_cast<const char*>(p.q) +
                          ((int64_t)b * p.q_stride_b + (int64_t)q_tile_row(qt) * p.q_stride_h) * 2;

@@ -161,11 +161,11 @@ def test_decode_tokens_of_infinitely_low_score(heads, num_ctas):
     torch.testing.assert_close(lse, lse_ref, **LSE_TOL)
 
 
-
 @pytest.mark.parametrize("heads,ps,stride", [(16, 64, 150_000_000), (20, 64, 120_000_000), (32, 1, 72_000_000),
-                                             (70, 64, 72_000_000)])
+                                             (70, 64, 72_000_000), (16, 64, 120_000_000), (40, 1, 64_000_000)])
 def test_decode_query_rows_beyond_32_bit_offsets(heads, ps, stride):
-    """Heads of a query so far apart that a tile of 16 or 32 of its rows spans more than 4 GiB."""
+    """Heads of a query so far apart that a tile of 16 or 32 of its rows spans more than 4 GiB, and (the last two) more
+    than 2 GiB, which unsigned offsets hold."""
     print(f"[decode query stride] heads={heads} ps={ps}", flush=True)
     lens = [300]
     case = make_decode_case(1, heads, ps, lens=lens, seed=heads)
