@@ -149,12 +149,13 @@ int mla_decode_plan(const int32_t *seq_lens, int32_t batch, int32_t page_size,
  *            ws_lse [ws_slots, heads] fp32
  *   out      [batch, heads, 512] strides (out_stride_b, out_stride_h)
  *   lse      [batch, heads] fp32 (row stride lse_stride_b) or NULL
- * heads is 1..1024: groups of at most 64 heads run one after another (each group reads the KV
- * again) and group g's partials occupy the workspace block [ws_slots, group heads, 512] that
+ * heads is 1..1024, in groups of at most 64; the groups of more than 64 heads run in one launch and share
+ * a plan range's KV through L2 (one launch per group, each reading the KV, where row offsets need 64 bits).
+ * Group g's partials occupy the workspace block [ws_slots, group heads, 512] that
  * starts at ws_o + ws_slots * 64 * g * 512 (ws_lse likewise), so a [ws_slots, heads, 512] buffer
- * holds them all; within a group, one wave per 16 heads (lanes past `heads` idle). page_size a power of
- * two; page ids outside [0, num_pages) are clamped into range.
- * Launches the split kernel on num_ctas CTAs, then the LSE merge kernel.
+ * holds them all. page_size a power of two; page ids outside [0, num_pages) are clamped into range.
+ * Launches the split kernel (a CTA per range and group, or one per compute unit that runs several
+ * ranges), then the LSE merge kernel.
  */
 int mla_decode_bf16(const void *q, int64_t q_stride_b, int64_t q_stride_h, const void *kv_pool,
                     int64_t kv_row_stride, int32_t num_pages, int32_t page_size,

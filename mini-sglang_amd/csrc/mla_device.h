@@ -90,9 +90,9 @@ __device__ __forceinline__ void dma16_saddr(const char* base, uint32_t voff, uin
 }
 // All column blocks of a token octet, one wave's 9 loads of a tile, as one statement that waits for its own base: a
 // base restored from a spill by a v_readlane right before the loads is then safe (with one statement per load, such a
-// restore loaded from a wild address). Block B lies 128 B bytes into the row and 4096 B bytes into the tile; the immediate offset is
-// added to the source and to the LDS address, so M0 steps by the difference. kNt: the non-temporal hint, for data
-// read once (streamed KV rows), so the caches keep the lines that are reused.
+// restore loaded from a wild address). Block i lies 128 i bytes into the row and 4096 i bytes into the tile; the
+// immediate offset is added to the source and to the LDS address, so M0 steps by the difference. kNt: the
+// non-temporal hint, for data read once (streamed KV rows), so the caches keep the lines that are reused.
 #define MLA_DMA_BLOCK(offset, hint) \
   "s_add_u32 m0, m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:" #offset hint "\n\t"
 #define MLA_DMA_OCTET(hint)                                                                                       \

@@ -144,8 +144,8 @@ __device__ __forceinline__ void mfma_pv(f32x16_t& o, const bf16x8& v, const u32x
 // keeps an output block in the vector registers and its MFMA in its slot
 __device__ __forceinline__ void pin_o(f32x16_t& o) { asm volatile("" : "+v"(o)); }
 
-// Pin a vector-ALU result to its place in the instruction stream: the empty volatile asm is
-// ordered with the MFMA asm statements, so the computation cannot drift into another slot.
+// Pin a vector-ALU result to its slot of the instruction stream: volatile asm statements keep their order, and the
+// slots' scheduling barriers keep each on its side.
 __device__ __forceinline__ void pin(float& x) { asm volatile("" : "+v"(x)); }
 __device__ __forceinline__ void pin(uint32_t& x) { asm volatile("" : "+v"(x)); }
 
@@ -175,10 +175,10 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int H = p.heads;
 
-  // ---- work item: request b, query block qb, head h (heads fastest). A request's last items (the latest query blocks, which see the most keys) are dispatched first,
-  // and of up to 64 requests the one with the most keys first: the long CTAs then do not run alone at the
-  // end (chunks of 531, 354 and 604 rows on prefixes of 2666, 197 and 296 keys, 64 heads: 119.3 us, 123.7 us in
-  // reverse request order)
+  // ---- work item: request b, query block qb, head h (heads fastest). A request's last items (the latest query blocks,
+  // which see the most keys) are dispatched first, and of up to 64 requests the one with the most keys first: the long
+  // CTAs then do not run alone at the end (chunks of 531, 354 and 604 rows on prefixes of 2666, 197 and 296 keys, 64
+  // heads: 119.3 us, 123.7 us in reverse request order)
   int b = -1, local = 0, q0 = 0, E = 0, L = 0;
   int item = (int)blockIdx.x;
   if (p.batch <= 64) {
@@ -504,10 +504,8 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
 
   f32x16_t O[4];
 #pragma unroll
-  for (int db = 0; db < 4; ++db)
-  O[db] = f32x16_t{};
+  for (int db = 0; db < 4; ++db) O[db] = f32x16_t{};
   float m_ref = -INFINITY, l_run = 0.f;
-  m_ref = -INFINITY, l_run = 0.f;
   f32x16_t sc[2];  // [parity]: scores of the stage being softmaxed / being computed
   u32x4 pb[2][2];  // [parity][ksp]: bf16 numerators P^T
   bf16x8 vb[kAV + 1];  // V^T operands in flight (the first kAV of a step are read by the step before)
@@ -536,7 +534,6 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
       if (8 * (i >> 2) + (i & 3) > lim) sv[i] = -INFINITY;
   };
   float negm = 0.f;  // -reference (log2 domain)
-  negm = 0.f;
   // reference of the wave's first stage: its exact row max
   auto init_ref = [&](f32x16_t& sv) __attribute__((always_inline)) {
     float m = sv[0];
@@ -637,7 +634,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
     asm volatile("v_max_f32 %1, %2, %3\n\tv_cmp_le_f32_e64 %0, %4, %1"
                  : "=s"(big), "=&v"(l_step_max) : "v"(l_step), "v"(l_step), "v"(kPLazyMax));
     if (big != 0) redo_stage(scs, pbw, l_step);
-  l_run += l_step;
+    l_run += l_step;
   };
 
   // step j <= W of a wave: the pipelined step. At j = 0 the value pass has no stage to add and is
@@ -660,8 +657,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
         // step 0 has no stage before it: its value pass multiplied zero numerators with whatever the V ring's
         // last slot held (NaN, if the LDS was left so), which must not count
 #pragma unroll
-        for (int db = 0; db < 4; ++db)
-  O[db] = f32x16_t{};
+        for (int db = 0; db < 4; ++db) O[db] = f32x16_t{};
       }
     } else {
       group_now(uk_c{}, uv_c{});
