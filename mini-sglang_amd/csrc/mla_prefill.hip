@@ -63,14 +63,13 @@ struct PShape<8> {
   static constexpr int kSync = 2, kDist = 4, kVLag = 0, kKRing = 7, kVRing = 7;
   static constexpr int kUnroll = 14;  // steps unrolled: whole rounds of the rings, and an even count (the score
                                       // and numerator registers alternate by step parity)
-  static constexpr int kWindow = 1023;  // stage sources held in LDS at a time (a whole number of entries
-                                       // per thread, with the one of dummy groups)
+  static constexpr int kWindow = 1024;  // stage sources held in LDS at a time
 };
 template <>
 struct PShape<4> {
   static constexpr int kSync = 1, kDist = 3, kVLag = 1, kKRing = 3, kVRing = 4;
   static constexpr int kUnroll = 12;
-  static constexpr int kWindow = 511;
+  static constexpr int kWindow = 512;
 };
 template <int NW>
 constexpr bool shape_ok() {
@@ -79,7 +78,7 @@ constexpr bool shape_ok() {
   // V live: j - 1 .. j + kDist - kVLag likewise
   return S::kKRing >= S::kDist + S::kSync - 1 && S::kVRing >= S::kDist - S::kVLag + 1 + S::kSync &&
          S::kUnroll % S::kKRing == 0 && S::kUnroll % S::kVRing == 0 && S::kUnroll % 2 == 0 &&
-         S::kWindow >= S::kUnroll + S::kVLag;  // a window holds the groups of a round of steps
+         S::kWindow > S::kUnroll + S::kVLag;  // a window holds the groups of a round of steps
 }
 static_assert(shape_ok<8>() && shape_ok<4>(), "ring lengths");
 // Wave-wide 1 KiB DMA loads of a stage: 12 of the K tile and 8 of the V tile; load i of a tile lands at i KiB.
@@ -169,7 +168,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
   constexpr int kKRingBytes = S::kKRing * kPKBytes;
   // the K ring, the V ring, then 1 KB that the loads of dummy DMA groups land in
   __shared__ __attribute__((aligned(1024))) char smem[kKRingBytes + S::kVRing * kPVBytes + 1024];
-  __shared__ __attribute__((aligned(16))) uint32_t s_src[S::kWindow + 1][4];  // K and V source of a window's stages
+  __shared__ __attribute__((aligned(16))) uint32_t s_src[S::kWindow][4];  // K and V source of a window's stages
 
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -285,8 +284,8 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
     return base + ((uint64_t)pid * page_bytes + (uint32_t)((t0 & ps_mask) * row_bytes));
   };
 
-  // ---- source addresses of the CTA's full stages, a window of them at a time: s_src[1 + i] is stage
-  // w0 + i's, and s_src[0] the first stage's, the source of dummy groups. The step loop fills the next window when a round of
+  // ---- source addresses of the CTA's full stages, a window of them at a time: s_src[i] is stage
+  // w0 + i's; stage n_defer's is the first stage's, the source of dummy groups. The step loop fills the next window when a round of
   // its steps would pass this one (every 500 steps and more: one drain of the loads). With a single window, CTAs of
   // more keys than it holds loaded each stage at once after a page-table read, with no loads ahead; single -> next
   // windows: 2048 rows on 20,000 keys, 8 heads 628 -> 370 us; 40 rows on 30,000, 64 heads 909 -> 483; four of 512
@@ -294,25 +293,25 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
   const int n_defer = min(nst, L >> 5);  // stages the pipelined step may load itself
   int w0 = 0;
   auto stage_window = [&](auto&& between) __attribute__((always_inline)) {
-    constexpr int kPer = (S::kWindow + 1) / (NW * 64);  // entries per thread
-    static_assert(kPer * NW * 64 == S::kWindow + 1, "every thread fills as many entries");
+    constexpr int kPer = S::kWindow / (NW * 64);  // entries per thread
+    static_assert(kPer * NW * 64 == S::kWindow, "every thread fills as many entries");
     int pid_u[kPer];
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-      const int e = threadIdx.x + NW * 64 * u, g = w0 + e - 1;
-      const int t0 = e > 0 && g < n_defer ? g * kPStage : 0;  // (an unconditional read: the first page's entry)
+      const int g = w0 + threadIdx.x + NW * 64 * u;
+      const int t0 = g < n_defer ? g * kPStage : 0;  // (an unconditional read: the first page's entry)
       pid_u[u] = p.page_table[(int64_t)b * p.pt_stride + (t0 >> p.log2_ps)];
     }
     between();
 #pragma unroll
     for (int u = 0; u < kPer; ++u) {
-      const int e = threadIdx.x + NW * 64 * u, g = w0 + e - 1;
-      if (e > 0 && g >= n_defer) continue;
-      const int t0 = e > 0 ? g * kPStage : 0;
+      const int i = threadIdx.x + NW * 64 * u, g = w0 + i;
+      if (g > n_defer) continue;
+      const int t0 = g < n_defer ? g * kPStage : 0;
       const uint32_t pid = (uint32_t)min(max(pid_u[u], 0), p.num_pages - 1);
       const uint64_t ka = (uint64_t)stage_src(kbase, pid, t0, kpage_bytes, krow_bytes);
       const uint64_t va = (uint64_t)stage_src(vbase, pid, t0, vpage_bytes, vrow_bytes);
-      *reinterpret_cast<MLA_LDS u32x4*>((MLA_LDS char*)s_src + 16 * e) =
+      *reinterpret_cast<MLA_LDS u32x4*>((MLA_LDS char*)s_src + 16 * i) =
           u32x4{(uint32_t)ka, (uint32_t)(ka >> 32), (uint32_t)va, (uint32_t)(va >> 32)};
     }
   };
@@ -402,17 +401,17 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
     constexpr int UK = decltype(uk_c)::value, UV = decltype(uv_c)::value;
     if constexpr (!kBoth) {
       const bool real = n_groups < n_defer;
-      dma_idx[0] = real ? n_groups - w0 + 1 : 0;
+      dma_idx[0] = min(n_groups, n_defer) - w0;
       dma_m0w[0] = real ? ring_lds + (UK >= 0 ? UK : n_groups % S::kKRing) * ring_stage : lds_dummy;
       dma_pst[0] = real ? 4 * 1024 : 0;
       if (__builtin_expect(!real && n_groups < nst, 0)) load_now(n_groups, k_wave, v_wave);
     } else {
       const int nv = n_groups - S::kVLag;
       const bool real_k = n_groups < n_defer, real_v = nv >= 0 && nv < n_defer;
-      dma_idx[0] = real_k ? n_groups - w0 + 1 : 0;
+      dma_idx[0] = min(n_groups, n_defer) - w0;
       dma_m0w[0] = real_k ? lds0 + wq * 1024 + (UK >= 0 ? UK : n_groups % S::kKRing) * kPKBytes : lds_dummy;
       dma_pst[0] = real_k ? 4 * 1024 : 0;
-      dma_idx[1] = real_v ? nv - w0 + 1 : 0;
+      dma_idx[1] = min(max(nv, 0), n_defer) - w0;
       dma_m0w[1] = real_v ? lds_v + wq * 1024 + (UV >= 0 ? UV : nv % S::kVRing) * kPVBytes : lds_dummy;
       dma_pst[1] = real_v ? 4 * 1024 : 0;
       if (__builtin_expect(!real_k && n_groups < nst, 0)) load_now(n_groups, true, false);
@@ -677,7 +676,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
   }
   for (int j0 = 0; j0 <= nst; j0 += S::kUnroll) {
     // this round's steps issue K stages j0 + kDist .. + kUnroll - 1 and V stages kVLag behind them
-    if (__builtin_expect(w0 + S::kWindow < min(j0 + S::kDist + S::kUnroll, n_defer), 0)) {
+    if (__builtin_expect(w0 + S::kWindow <= min(j0 + S::kDist + S::kUnroll - 1, n_defer), 0)) {
       barrier_lds();  // every wave is done with the window's entries
       w0 = j0 + S::kDist - S::kVLag;
       // (a wait of its own: page-table reads that a path leaves open make every step wait for all its loads)
