@@ -78,7 +78,7 @@ constexpr bool shape_ok() {
   // V live: j - 1 .. j + kDist - kVLag likewise
   return S::kKRing >= S::kDist + S::kSync - 1 && S::kVRing >= S::kDist - S::kVLag + 1 + S::kSync &&
          S::kUnroll % S::kKRing == 0 && S::kUnroll % S::kVRing == 0 && S::kUnroll % 2 == 0 &&
-         S::kWindow > S::kUnroll + S::kVLag;  // a window holds the groups of a round of steps
+         S::kWindow > S::kUnroll + S::kVLag;  // a window holds the groups of kUnroll steps
 }
 static_assert(shape_ok<8>() && shape_ok<4>(), "ring lengths");
 // Wave-wide 1 KiB DMA loads of a stage: 12 of the K tile and 8 of the V tile; load i of a tile lands at i KiB.
@@ -284,12 +284,12 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
     return base + ((uint64_t)pid * page_bytes + (uint32_t)((t0 & ps_mask) * row_bytes));
   };
 
-  // ---- source addresses of the CTA's full stages, a window of them at a time: s_src[i] is stage
-  // w0 + i's; stage n_defer's is the first stage's, the source of dummy groups. The step loop fills the next window when a round of
-  // its steps would pass this one (every 500 steps and more: one drain of the loads). With a single window, CTAs of
-  // more keys than it holds loaded each stage at once after a page-table read, with no loads ahead; single -> next
-  // windows: 2048 rows on 20,000 keys, 8 heads 628 -> 370 us; 40 rows on 30,000, 64 heads 909 -> 483; four of 512
-  // rows on 16,000 1631 -> 1238; 2048 rows on 40,000 (256-row CTAs) 3247 -> 2795.
+  // ---- source addresses of the CTA's full stages, a window of them at a time: s_src[i] is stage w0 + i's; stage
+  // n_defer's is the first stage's, the source of dummy groups. The step loop fills the next window when its next
+  // kUnroll steps would pass this one (every 500 steps and more: one drain of the loads). With a single window, CTAs
+  // of more keys than it holds loaded each stage at once after a page-table read, with no loads ahead; single -> next
+  // windows: 2048 rows on 20,000 keys, 8 heads 628 -> 366 us; 40 rows on 30,000, 64 heads 909 -> 480; four of 512
+  // rows on 16,000 1662 -> 1196; 2048 rows on 40,000 (256-row CTAs) 3293 -> 2860.
   const int n_defer = min(nst, L >> 5);  // stages the pipelined step may load itself
   int w0 = 0;
   auto stage_window = [&](auto&& between) __attribute__((always_inline)) {
@@ -675,7 +675,7 @@ __global__ __launch_bounds__(NW * 64, 2) void mla_prefill_kernel(const PrefillPa
     for (int st = 0; st < kAV; ++st) vb[st] = vop(0, st);
   }
   for (int j0 = 0; j0 <= nst; j0 += S::kUnroll) {
-    // this round's steps issue K stages j0 + kDist .. + kUnroll - 1 and V stages kVLag behind them
+    // the next kUnroll steps issue K stages j0 + kDist .. + kUnroll - 1 and V stages kVLag behind them
     if (__builtin_expect(w0 + S::kWindow <= min(j0 + S::kDist + S::kUnroll - 1, n_defer), 0)) {
       barrier_lds();  // every wave is done with the window's entries
       w0 = j0 + S::kDist - S::kVLag;
